@@ -97,12 +97,24 @@ __device__ __forceinline__ void wait_groups(int k) {
 // straight from the packed rows with ds_read_b64_tr_b4 (16 tokens of one latent
 // dim per lane), widens the e2m1 codes to bf16 unscaled, and folds each token's
 // e8m0 block scale into P instead: P'_j = P * 2^(e[t, j] - E_ref) for MX block j,
-// with P = 2^(s - m_ref) in f32 shared through LDS and E_ref a per-item
-// reference exponent; O^T is rescaled by 2^(E_ref - 127) at the end.  PV runs on
-// 16x16x32 bf16 MFMAs.  The LDS this frees lets two work-groups share a CU.
-// A tile max more than kRebase above m_ref, or (fp4 V) a V block exponent more
-// than kVScaleSpan above E_ref, restarts the item from a higher reference
-// (block-wide vote), so neither the accumulators nor P' can overflow.
+// with P = 2^(s - m_ref) shared through LDS as the bf16 the MFMA takes and E_ref
+// a per-item reference exponent; O^T is rescaled by 2^(E_ref - 127) at the end.
+// PV runs on 16x16x32 bf16 MFMAs.  The LDS this frees lets two work-groups share
+// a CU.  This path is bound by instruction issue, not by its bytes (256 x 8192
+// contiguous tokens of 306 B: 4.3 TB/s where the fp8 rows reach 6.7), so the
+// tile does no work twice: P is packed once by the wave that scores it, not by
+// every wave that reads it; the block exponents become 16-bit steps in a small
+// per-wave table, one saturating subtract per pair of P' instead of a byte
+// permute, a multiply-add and a max; and the references are checked once per
+// item instead of by a vote per tile.  VALU per wave and tile 309 -> 192;
+// 256 x 8192 149.7 -> 129.1 us a call, 128 x 4096 scattered 59.4 -> 56.1,
+// 4 x 8192 20.1 -> 19.2.
+// fp8 V: a tile max more than kRebase above m_ref restarts the item from a
+// higher reference (a block-wide vote per tile).  bf16 PV: a score, or (fp4 V) a
+// V block exponent more than kVScaleSpan above E_ref, found so far above its
+// reference anywhere in a pass runs the item again from the maxima of the whole
+// item (nothing of the first pass is kept).  Either way neither the accumulators
+// nor P' of the pass that counts can overflow.
 // ============================================================================
 // KF / VF: 0 / 0 fp8 K = V, 1 / 2 fp4 K = V, 1 / 1 fp4 K + fp8 V, 2 / 3 bf16 K =
 // V (a16w16: 1152-byte rows, V = their first 512 dims; QK and PV on 16x16x32
@@ -134,15 +146,16 @@ struct H16 {
   static constexpr int NA = (NW + NRW - 1) / NRW;              // windows per row wave: NA or NA - 1
   static constexpr int NAW = NW % NRW == 0 ? NRW : NW % NRW;   // row waves (from RW0) that issue NA
   static constexpr bool VB16 = VF == 2;                        // fp4 V, bf16 PV from registers
-  static constexpr bool P32 = VF >= 2;                         // P shared as f32 [head][token] (bf16 PV)
-  static constexpr int PST = 68;                               // f32 P row stride (P32): 64 tokens + 4
+  static constexpr bool PB = VF >= 2;                          // P shared as bf16 [head][token] (bf16 PV)
+  static constexpr int PST = 144;                              // its row stride in bytes: 64 tokens + 16
   static constexpr int NSL = 2 * S;                            // slot stages (slots lead rows by S tiles)
   static constexpr int OFF_SLOT = S * STAGE;                   // [NSL][64] int32 cache slots
   static constexpr int SCST = kScWin * 256;                    // e8m0 stage: [5][64 tokens] dwords
   static constexpr int OFF_SC = OFF_SLOT + NSL * 256;          // [S] e8m0 stages (KF == 1)
   static constexpr int OFF_P = OFF_SC + (KF == 1 ? S * SCST : 0);
-  static constexpr int P_BYTES = P32 ? 16 * PST * 4 : 2 * 4 * 16 * 16;  // f32 [h][token] | fp8 [term][g][h][16]
-  static constexpr int OFF_PS = OFF_P + P_BYTES;               // [g][h] e8m0 B scales
+  static constexpr int P_BYTES = PB ? 16 * PST : 2 * 4 * 16 * 16;  // bf16 [h][token] | fp8 [term][g][h][16]
+  static constexpr int OFF_ET = OFF_P + P_BYTES;               // fp4 V: [wave][block][64 tokens] u16 exponent steps
+  static constexpr int OFF_PS = OFF_ET + (VB16 ? 4 * 4 * 128 : 0);  // [g][h] e8m0 B scales
   static constexpr int OFF_X = OFF_PS + 64;                    // [4][16] f32 exchange
   static constexpr int OFF_E = OFF_X + 256;                    // [4] int exchange (V block exponents)
   static constexpr int OFF_VOTE = OFF_E + 16;
@@ -517,6 +530,7 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
   float m_ref = 0.f, m_seen = neg_inf(), l_part = 0.f;
   bool have_ref = false;
   int e_ref = 127, e_seen = 0;  // fp4 V: reference and running max of the V block exponents
+  // (m_seen: fp8 V the wave's ceil max of a head, bf16 PV the lane's raw score max)
 
   auto prologue = [&](bool slots_issued, bool quant) __attribute__((always_inline)) {
     if (!slots_issued) {
@@ -539,6 +553,31 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
   // ---- main loop ---------------------------------------------------------------
   int8_t* vote = reinterpret_cast<int8_t*>(smem + C::OFF_VOTE);
   float* xch = reinterpret_cast<float*>(smem + C::OFF_X);
+  // bf16 PV: the item's references from the maxima seen so far (raw scores,
+  // V block exponents), over the lanes of a head and the waves
+  auto set_refs = [&]() __attribute__((always_inline)) {
+    float mx = fmaxf(m_seen, shfl_xor_f(m_seen, 16));
+    mx = __builtin_ceilf(fmaxf(mx, shfl_xor_f(mx, 32)) * c);
+    int* ex = reinterpret_cast<int*>(smem + C::OFF_E);
+    const int e_w = C::VB16 ? wave_max(e_seen) : 0;
+    if (g == 0) xch[16 * w + l16] = mx;
+    if (C::VB16 && lane == 0) ex[w] = e_w;
+    lds_barrier();
+    m_ref = fmaxf(fmaxf(xch[l16], xch[16 + l16]), fmaxf(xch[32 + l16], xch[48 + l16]));
+    if constexpr (C::VB16) e_ref = max(max(ex[0], ex[1]), max(ex[2], ex[3]));
+  };
+  // fp4 V: the wave's exponent steps of one tile, from its e8m0 dword plane
+  auto scale_steps = [&](const uint8_t* sct) __attribute__((always_inline)) {
+    const uint32_t ed = *reinterpret_cast<const uint32_t*>(sct + 256 * w + 4 * lane);
+    const u16x2 top = (u16x2)(unsigned short)(e_ref + kVScaleSpan);
+    const u16x2 d01 = (top - __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(0u, ed, 0x0C010C00u))) << (u16x2)(unsigned short)7;
+    const u16x2 d23 = (top - __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(0u, ed, 0x0C030C02u))) << (u16x2)(unsigned short)7;
+    uint16_t* et = reinterpret_cast<uint16_t*>(smem + C::OFF_ET + 512 * w) + lane;
+    et[0] = d01[0];
+    et[64] = d01[1];
+    et[128] = d23[0];
+    et[192] = d23[1];
+  };
   bool slots_issued = true;  // by the early issue above; a restart issues them again
   bool q_pending = QB;       // Q is quantized in the first prologue only
   for (;;) {
@@ -562,10 +601,15 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
       // e8m0 of (token t, block j): byte j & 3 of dword (j >> 2, t) at 256 (j >> 2)
       // + 4 t (j < 16), byte j - 14 of dword (4, t) (j = 16, 17)
       const uint8_t* sct = smem + C::OFF_SC + st * C::SCST;
+      if constexpr (C::VB16) {
+        // this wave's V blocks 4w .. 4w + 3: (e_ref + kVScaleSpan - e) << 7 of
+        // token `lane`, four 16-bit steps, into the wave's own table; PV takes
+        // them off P's bf16 exponent field with one saturating subtract
+        if (have_ref) scale_steps(sct);
+      }
 
       // ---- scores: rows i = l16 of this wave's slice, 16x16x128 MFMAs ----------
       v4f s = v4f{0.f, 0.f, 0.f, 0.f};
-      int e_w = 0;  // fp4 V: max V block exponent of this wave's 16 tokens
       {
         // all fragment reads first, then the MFMA chain
         const uint8_t* kp = kt + tok_of(w, l16) * C::KST;
@@ -598,37 +642,58 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
           }
 #pragma unroll
           for (int ks = 0; ks < 5; ++ks) s = mfma16_f4f8(ka[ks], ksc[ks], qv[ks], s);
-          if constexpr (C::VB16) {  // V blocks 0..15 are K blocks 4ks + g, ks < 4
-            e_w = wave_max(max(max(ksc[0], ksc[1]), max(ksc[2], ksc[3])));
-            e_seen = max(e_seen, e_w);
-          }
+          if constexpr (C::VB16)  // V blocks 0..15 are K blocks 4ks + g, ks < 4
+            e_seen = max(max(e_seen, max(ksc[0], ksc[1])), max(ksc[2], ksc[3]));
         }
       }
-      // s[r] = score(token tok_of(w, 4g + r), head l16)
-      float sv[4];
-      float mx = neg_inf();
+      if constexpr (C::PB) {
+        // s[r] = score(token tok_of(w, 4g + r), head l16); positions past the
+        // item repeat its last token, so they may enter the maxima
+        m_seen = fmaxf(fmaxf(m_seen, fmaxf(s[0], s[1])), fmaxf(s[2], s[3]));
+        if (!have_ref) {  // first tile of the first pass
+          set_refs();
+          if constexpr (C::VB16) scale_steps(sct);
+          have_ref = true;
+        }
+        // P = 2^(s - m_ref); its row sum in f32, and as bf16 for the PV product
+        // (fp4 V: with kVScaleSpan added to the exponent, see scale_steps)
+        float pw[4];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        sv[r] = tok_of(w, 4 * g + r) < nval ? s[r] * c : neg_inf();
-        mx = fmaxf(mx, sv[r]);
-      }
-      mx = fmaxf(mx, shfl_xor_f(mx, 16));
-      mx = fmaxf(mx, shfl_xor_f(mx, 32));
-      const float m_w = mx == neg_inf() ? neg_inf() : __builtin_ceilf(mx);
-      m_seen = fmaxf(m_seen, m_w);
-      int* ex = reinterpret_cast<int*>(smem + C::OFF_E);
-      if (!have_ref) {  // first tile of the first pass: references = tile maxima over the waves
-        if (g == 0) xch[16 * w + l16] = m_w;
-        if (C::VB16 && lane == 0) ex[w] = e_w;
-        lds_barrier();
-        m_ref = fmaxf(fmaxf(xch[l16], xch[16 + l16]), fmaxf(xch[32 + l16], xch[48 + l16]));
-        if constexpr (C::VB16) e_ref = max(max(ex[0], ex[1]), max(ex[2], ex[3]));
-        have_ref = true;
-      }
-      const bool over = __any(m_w > m_ref + kRebase) || (C::VB16 && e_w > e_ref + kVScaleSpan);
-      if (lane == 0) vote[w] = over ? 1 : 0;
-
-      if constexpr (!C::P32) {
+        for (int r = 0; r < 4; ++r) pw[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c, -m_ref));
+        if (nval < kTile) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) pw[r] = tok_of(w, 4 * g + r) < nval ? pw[r] : 0.f;
+        }
+        l_part += (pw[0] + pw[1]) + (pw[2] + pw[3]);
+        u16x2 p01 = __builtin_bit_cast(u16x2, pack_bf16x2(pw[0], pw[1]));
+        u16x2 p23 = __builtin_bit_cast(u16x2, pack_bf16x2(pw[2], pw[3]));
+        if constexpr (C::VB16) {
+          p01 += (u16x2)(unsigned short)(kVScaleSpan << 7);
+          p23 += (u16x2)(unsigned short)(kVScaleSpan << 7);
+        }
+        *reinterpret_cast<uint2*>(smem + C::OFF_P + l16 * C::PST + 2 * tok_of(w, 4 * g)) =
+            make_uint2(__builtin_bit_cast(uint32_t, p01), __builtin_bit_cast(uint32_t, p23));
+      } else {
+        // s[r] = score(token tok_of(w, 4g + r), head l16)
+        float sv[4];
+        float mx = neg_inf();
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          sv[r] = tok_of(w, 4 * g + r) < nval ? s[r] * c : neg_inf();
+          mx = fmaxf(mx, sv[r]);
+        }
+        mx = fmaxf(mx, shfl_xor_f(mx, 16));
+        mx = fmaxf(mx, shfl_xor_f(mx, 32));
+        const float m_w = mx == neg_inf() ? neg_inf() : __builtin_ceilf(mx);
+        m_seen = fmaxf(m_seen, m_w);
+        if (!have_ref) {  // first tile of the first pass: references = tile maxima over the waves
+          if (g == 0) xch[16 * w + l16] = m_w;
+          lds_barrier();
+          m_ref = fmaxf(fmaxf(xch[l16], xch[16 + l16]), fmaxf(xch[32 + l16], xch[48 + l16]));
+          have_ref = true;
+        }
+        const bool over = __any(m_w > m_ref + kRebase);
+        if (lane == 0) vote[w] = over ? 1 : 0;
         // P' = 2^(s - m_w) * 2^8 (two fp8 terms); B scale 2^(m_w - m_ref - 8)
         const float mw = m_w == neg_inf() ? m_ref : m_w;
         const float dm = fminf(fmaxf(mw - m_ref, -160.f), 160.f);
@@ -645,21 +710,13 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
         *reinterpret_cast<uint32_t*>(pl) = hi;
         *reinterpret_cast<uint32_t*>(pl + 4 * 256) = lo;
         if (g == 0) smem[C::OFF_PS + 16 * w + l16] = (uint8_t)min(max((int)dm - 8 + 127, 0), 254);
-      } else {
-        // f32 P = 2^(s - m_ref), row-major [head][token]
-        float pw[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          pw[r] = __builtin_amdgcn_exp2f(fminf(sv[r] - m_ref, 120.f));
-          l_part += pw[r];
-        }
-        *reinterpret_cast<float4*>(reinterpret_cast<float*>(smem + C::OFF_P) + l16 * C::PST + tok_of(w, 4 * g)) =
-            make_float4(pw[0], pw[1], pw[2], pw[3]);
       }
-      lds_barrier();  // (2) P, its scales and the votes visible
-      if (__builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(vote)) != 0) {
-        restart = true;
-        break;
+      lds_barrier();  // (2) P (fp8 V: its scales and the votes) visible
+      if constexpr (!C::PB) {
+        if (__builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(vote)) != 0) {
+          restart = true;
+          break;
+        }
       }
 
       // ---- O^T[dims 128w ..] += V^T . P^T ---------------------------------------
@@ -670,15 +727,10 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
         // element i = element j & 3 of source lane 4i + (j >> 2); source lane
         // s reads token 8g + 4u + (s >> 2), dims 16dt + 4(s & 3) .. +3, so read
         // u gives lane m tokens 8g + 4u .. +3 of dim 16dt + m.
-        const float* prow = reinterpret_cast<const float*>(smem + C::OFF_P) + l16 * C::PST;
+        const uint8_t* prow = smem + C::OFF_P + l16 * C::PST + 16 * g;
         v8bf pb[2];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const float4 pa = *reinterpret_cast<const float4*>(prow + 32 * h + 8 * g);
-          const float4 pc = *reinterpret_cast<const float4*>(prow + 32 * h + 8 * g + 4);
-          pb[h] = __builtin_bit_cast(v8bf, make_uint4(pack_bf16x2(pa.x, pa.y), pack_bf16x2(pa.z, pa.w),
-                                                      pack_bf16x2(pc.x, pc.y), pack_bf16x2(pc.z, pc.w)));
-        }
+        for (int h = 0; h < 2; ++h) pb[h] = __builtin_bit_cast(v8bf, *reinterpret_cast<const uint4*>(prow + 64 * h));
         const uint32_t vb = lds0 + st * C::STAGE + (8 * g + (l16 >> 2)) * C::KST + 2 * (128 * w + 4 * (l16 & 3));
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) {
@@ -731,56 +783,27 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
         // tile whose source lane m' reads row T(g, m'), so result lane m gets
         // dim 16dt + m of those 16 tokens, widened to bf16 at unit scale.
         // P'^T: P of the same tokens times 2^(e[t, j] - E_ref) for the MX block
-        // j of the tile's dims, in bf16.  The shift is applied in one step: a
-        // small P whose token has a large block exponent would lose its mantissa
-        // to f32 subnormals if P were scaled by 2^-E_ref first.
-        const float* prow = reinterpret_cast<const float*>(smem + C::OFF_P) + l16 * C::PST;
-        float pv[16];
-        {
-          const float4 p0 = *reinterpret_cast<const float4*>(prow + 8 * g);
-          const float4 p1 = *reinterpret_cast<const float4*>(prow + 8 * g + 4);
-          const float4 p2 = *reinterpret_cast<const float4*>(prow + 32 + 8 * g);
-          const float4 p3 = *reinterpret_cast<const float4*>(prow + 36 + 8 * g);
-          const float pa[16] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w,
-                                p2.x, p2.y, p2.z, p2.w, p3.x, p3.y, p3.z, p3.w};
-#pragma unroll
-          for (int k = 0; k < 16; ++k) pv[k] = pa[k];
-        }
+        // j of the tile's dims, in bf16: P's exponent field (raised by
+        // kVScaleSpan) less the token's step of scale_steps, per 16-bit half.
+        // The saturation turns a P' below the normal range into 0; P <=
+        // 2^kRebase and e <= E_ref + kVScaleSpan (else the pass is run again)
+        // keep it finite.
+        const uint8_t* prow = smem + C::OFF_P + l16 * C::PST + 16 * g;
+        const uint4 p0 = *reinterpret_cast<const uint4*>(prow), p1 = *reinterpret_cast<const uint4*>(prow + 64);
+        const uint32_t pq[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
         const int trow = l16 < 8 ? 8 * g + l16 : 24 + 8 * g + l16;
         const uint32_t va = lds0 + st * C::STAGE + trow * C::KST + 64 * w;
-        // dword (w, t): the e8m0 of this wave's blocks 4w .. 4w + 3 (dims 128w ..)
-        const int* se = reinterpret_cast<const int*>(sct) + 64 * w;
-        const int4 e0 = *reinterpret_cast<const int4*>(se + 8 * g);
-        const int4 e1 = *reinterpret_cast<const int4*>(se + 8 * g + 4);
-        const int4 e2 = *reinterpret_cast<const int4*>(se + 32 + 8 * g);
-        const int4 e3 = *reinterpret_cast<const int4*>(se + 36 + 8 * g);
-        const uint32_t ed[16] = {(uint32_t)e0.x, (uint32_t)e0.y, (uint32_t)e0.z, (uint32_t)e0.w,
-                                 (uint32_t)e1.x, (uint32_t)e1.y, (uint32_t)e1.z, (uint32_t)e1.w,
-                                 (uint32_t)e2.x, (uint32_t)e2.y, (uint32_t)e2.z, (uint32_t)e2.w,
-                                 (uint32_t)e3.x, (uint32_t)e3.y, (uint32_t)e3.z, (uint32_t)e3.w};
-        // P of tokens (k, k + 1) as a bf16 pair with E_ref taken off both
-        // exponent fields (16-bit lanes, mod 2^16); block jl then adds e << 7
-        // per half, which is the exact bf16 of P 2^(e - E_ref) while that
-        // stays a normal number.  P <= 2^kRebase and e <= E_ref + kVScaleSpan
-        // keep every sum below 2^15, so a negative 16-bit result means the
-        // scaled P fell below the normal range: it becomes 0.
-        u16x2 pq[8];
-        const u16x2 eoff = (u16x2)(unsigned short)(e_ref << 7);
+        const uint8_t* et = smem + C::OFF_ET + 512 * w + 16 * g;
 #pragma unroll
-        for (int k = 0; k < 16; k += 2) pq[k / 2] = __builtin_bit_cast(u16x2, pack_bf16x2(pv[k], pv[k + 1])) - eoff;
-#pragma unroll
-        for (int jl = 0; jl < 4; ++jl) {  // block 4w + jl (dims 32(4w + jl) ..): byte jl
+        for (int jl = 0; jl < 4; ++jl) {  // block 4w + jl (dims 32(4w + jl) ..)
+          const uint4 d0 = *reinterpret_cast<const uint4*>(et + 128 * jl);
+          const uint4 d1 = *reinterpret_cast<const uint4*>(et + 128 * jl + 64);
+          const uint32_t dq[8] = {d0.x, d0.y, d0.z, d0.w, d1.x, d1.y, d1.z, d1.w};
           uint32_t bw[8];
 #pragma unroll
-          for (int k = 0; k < 16; k += 2) {
-            // byte jl of tokens k and k + 1 into the low bytes of the two halves
-            const uint32_t x = __builtin_amdgcn_perm(ed[k + 1], ed[k], jl | 0x0C00u | ((4u + jl) << 16) | 0x0C000000u);
-            // (e << 7) + P per half in one packed multiply-add (the compiler
-            // would shift and add); its operands and result are plain VGPRs
-            uint32_t y;
-            asm("v_pk_mad_u16 %0, %1, %2, %3" : "=v"(y) : "v"(x), "s"(0x00800080u), "v"(pq[k / 2]));
-            bw[k / 2] = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(s16x2, y), (s16x2)0));
-          }
+          for (int k = 0; k < 8; ++k)
+            bw[k] = __builtin_bit_cast(uint32_t, __builtin_elementwise_sub_sat(__builtin_bit_cast(u16x2, pq[k]),
+                                                                               __builtin_bit_cast(u16x2, dq[k])));
           const v8bf b0 = __builtin_bit_cast(v8bf, make_uint4(bw[0], bw[1], bw[2], bw[3]));
           const v8bf b1 = __builtin_bit_cast(v8bf, make_uint4(bw[4], bw[5], bw[6], bw[7]));
 #pragma unroll
@@ -800,16 +823,24 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
         }
       }
     }
+    if constexpr (C::PB) {
+      // a score or V block exponent too far above its reference anywhere in
+      // the pass: run the item again from the maxima of the whole item
+      const bool over = ntiles > 0 && (__any(m_seen * c > m_ref + kRebase) ||
+                                       (C::VB16 && __any(e_seen > e_ref + kVScaleSpan)));
+      if (lane == 0) vote[w] = over ? 1 : 0;
+      lds_barrier();
+      restart = __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(vote)) != 0;
+    }
     if (!restart) break;
     // drain the ring (the prologue reuses it); m_ref = running max over the waves
     wait_vmcnt<0>();
-    if (g == 0) xch[16 * w + l16] = m_seen;
-    if (C::VB16 && lane == 0) reinterpret_cast<int*>(smem + C::OFF_E)[w] = e_seen;
-    lds_barrier();
-    m_ref = fmaxf(fmaxf(xch[l16], xch[16 + l16]), fmaxf(xch[32 + l16], xch[48 + l16]));
-    if constexpr (C::VB16) {
-      const int* ex = reinterpret_cast<const int*>(smem + C::OFF_E);
-      e_ref = max(max(ex[0], ex[1]), max(ex[2], ex[3]));
+    if constexpr (C::PB) {
+      set_refs();
+    } else {
+      if (g == 0) xch[16 * w + l16] = m_seen;
+      lds_barrier();
+      m_ref = fmaxf(fmaxf(xch[l16], xch[16 + l16]), fmaxf(xch[32 + l16], xch[48 + l16]));
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = v4f{0.f, 0.f, 0.f, 0.f};
