@@ -138,10 +138,10 @@ struct H16 {
   static constexpr int S = KF != 1 ? 2 : (VF == 1 ? 2 : 3);
   static constexpr int BLOCKS_PER_CU = (VF == 1 || KF == 2) ? 1 : 2;
   // DMA issue: waves RW0..3 gather rows.  fp4 K + fp8 V: wave 0 gathers the
-  // 18 scale bytes of every token (SCW = 1); fp4 K = V: every wave gathers rows
-  // and scale dword columns j = w + 4k (SCW = 4), so no wave issues a long burst
+  // scales of every token.  fp4 K = V: every wave gathers rows and one scale
+  // dword column, wave 3, which has a row window less, a second one, so every
+  // wave issues the same number
   static constexpr int RW0 = (KF == 1 && VF == 1) ? 1 : 0;
-  static constexpr int SCW = KF == 0 ? 0 : (VF == 1 ? 1 : 4);
   static constexpr int NRW = 4 - RW0;
   static constexpr int NA = (NW + NRW - 1) / NRW;              // windows per row wave: NA or NA - 1
   static constexpr int NAW = NW % NRW == 0 ? NRW : NW % NRW;   // row waves (from RW0) that issue NA
@@ -233,7 +233,9 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
     if ((int)blockIdx.x >= plan[0]) return;
     it = reinterpret_cast<const int4*>(plan + kPlanHeader)[blockIdx.x];
   }
-  const int b = it.x, t_beg = it.y, t_end = it.z, slot = it.w;
+  // the item is the work-group's: its fields in scalar registers
+  const int b = __builtin_amdgcn_readfirstlane(it.x), t_beg = __builtin_amdgcn_readfirstlane(it.y);
+  const int t_end = __builtin_amdgcn_readfirstlane(it.z), slot = __builtin_amdgcn_readfirstlane(it.w);
   const int ntok = t_end - t_beg;
   const int ntiles = (ntok + kTile - 1) / kTile;
 
@@ -244,50 +246,100 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
   auto tok_of = [](int gg, int i) { return 16 * gg + i; };  // tile token of row i of wave gg's slice
 
   // ---- ring issue ----------------------------------------------------------
-  // slots of tile t live in slot stage t % NSL
-  auto slot_of = [&](int t, int tok) -> int __attribute__((always_inline)) {
-    if constexpr (IDX) return reinterpret_cast<const int*>(smem + C::OFF_SLOT + (t % C::NSL) * 256)[tok];
+  // Tile t's rows live in ring stage t % S, its slots in slot stage t % NSL;
+  // the callers carry both indices (no division per tile).
+  auto slot_of = [&](int t, int ss, int tok) __attribute__((always_inline)) -> int {
+    if constexpr (IDX) return reinterpret_cast<const int*>(smem + C::OFF_SLOT + ss * 256)[tok];
     else return min(t_beg + kTile * t + tok, t_end - 1);
   };
-  auto issue_slots = [&](int t) __attribute__((always_inline)) {  // wave 0: the 64 slots of tile t (positions clamped into the item)
+  auto issue_slots = [&](int t, int ss) __attribute__((always_inline)) {  // wave 0: the 64 slots of tile t (positions clamped into the item)
     if constexpr (IDX) {
       if (w == 0) {
         const int pos = min(t_beg + kTile * t + lane, t_end - 1);
-        dma4_to_lds(p.kv_indices + pos, lds0 + C::OFF_SLOT + (t % C::NSL) * 256);
+        dma4_to_lds(p.kv_indices + pos, lds0 + C::OFF_SLOT + ss * 256);
       }
     }
   };
-  auto issue_rows = [&](int t) __attribute__((always_inline)) {  // row waves: windows u = (w - RW0) + NRW k of tile t
-    if (w < C::RW0) return;
-    const int st = t % C::S;
-    const uint32_t sbase = lds0 + st * C::STAGE;
-    // all slot reads first: each DMA below is an asm barrier for memory ops
-    int sl[C::NA], co[C::NA];
+  // Contiguous rows of a tile that lies whole inside the item are addressed as
+  // one scalar base per tile plus offsets that stay in registers (below 2^31:
+  // the stride test), which takes the address arithmetic, a quarter-rate
+  // multiply-add per window, out of the loop.  With the ring indices carried
+  // and the DMAs issued four to an M0 save, 256 x 8192 mxfp4 129.1 -> 123.1 us a
+  // call; scattered rows gain from the latter two (128 x 4096 56.1 -> 53.4)
+  // (a16w8, whose two fp8 terms of Q leave no registers for them, computes
+  // every address)
+  constexpr int64_t kFarStride = 1 << 24;
+  constexpr bool kNear = !IDX && QM != 2;
+  const bool near_rows = kNear && p.k_row_stride <= kFarStride && (KF != 1 || p.k_scale_stride <= kFarStride);
+  uint32_t voff[C::VW == 0 && (kNear || QM == 2) ? C::NA : 1];
+  if constexpr (C::VW == 0 && (kNear || QM == 2)) {
 #pragma unroll
     for (int k = 0; k < C::NA; ++k) {
-      const int u = (w - C::RW0) + C::NRW * k;
-      if (u < C::KW) {
-        const int e = 64 * u + lane;  // 16-B chunk index within the stage
-        const int tok = e / C::KCPR, ch = e - tok * C::KCPR;
-        sl[k] = slot_of(t, tok);
-        co[k] = 16 * min(ch, C::KCH - 1);
-      } else if (u < C::NW) {
-        const int e = 64 * (u - C::KW) + lane;
-        const int tok = e / C::VCPR, ch = e - tok * C::VCPR;
-        sl[k] = slot_of(t, tok);
-        co[k] = 16 * min(ch, 31);
-      }
+      const int e = 64 * (w + 4 * k) + lane, tok = e / C::KCPR, ch = e - tok * C::KCPR;
+      voff[k] = (kNear ? (uint32_t)tok * (uint32_t)p.k_row_stride : 0u) + (uint32_t)(16 * min(ch, C::KCH - 1));
     }
+  }
+  auto issue_rows = [&](int t, int st, int ss) __attribute__((always_inline)) {
+    if constexpr (C::VW == 0) {
+      // windows u = w + 4k of the stage; the last one (k = NA - 1) on waves below NAW
+      static_assert(C::RW0 == 0, "every wave gathers rows");
+      const uint32_t base = __builtin_amdgcn_readfirstlane(lds0 + st * C::STAGE + 1024 * w);
+      if constexpr (kNear) {
+        if (near_rows && kTile * (t + 1) <= ntok) {
+          const uint8_t* sb = p.k_cache + (int64_t)(t_beg + kTile * t) * p.k_row_stride;
+          dma16_windows<0, C::NA - 1>(base, [&](auto k) __attribute__((always_inline)) { return voff[decltype(k)::value]; }, sb);
+          if (w < C::NAW) dma16_windows<C::NA - 1, C::NA>(base, [&](auto k) __attribute__((always_inline)) { return voff[decltype(k)::value]; }, sb);
+          return;
+        }
+      }
+      // all slot reads first (each DMA block below is an asm barrier for memory
+      // ops), the addresses as each block needs them
+      int sl[C::NA];
 #pragma unroll
-    for (int k = 0; k < C::NA; ++k) {
-      const int u = (w - C::RW0) + C::NRW * k;
-      // slot x stride in one v_mad_u64_u32 (both below 2^31, checked on the host)
-      if (u < C::KW)
-        dma16_to_lds_nt(p.k_cache + ((uint64_t)(uint32_t)sl[k] * (uint32_t)p.k_row_stride + (uint32_t)co[k]),
-                     sbase + 1024 * u);
-      else if (u < C::NW)
-        dma16_to_lds_nt(p.v_cache + ((uint64_t)(uint32_t)sl[k] * (uint32_t)p.v_row_stride + (uint32_t)co[k]),
-                     sbase + 1024 * u);
+      for (int k = 0; k < C::NA; ++k) sl[k] = slot_of(t, ss, min(64 * (w + 4 * k) + lane, kTile * C::KCPR - 1) / C::KCPR);
+      auto row_addr = [&](auto kt) __attribute__((always_inline)) {
+        constexpr int k = decltype(kt)::value;
+        // 16-B chunk of the row (the last one pads)
+        uint32_t co = (uint32_t)(16 * min((64 * (w + 4 * k) + lane) % C::KCPR, C::KCH - 1));
+        if constexpr (QM == 2) {  // a 32-bit offset kept per window, not the 64-bit base + offset
+          asm volatile("" : "+v"(voff[k]));
+          co = voff[k];
+        }
+        // slot x stride in one v_mad_u64_u32 (both below 2^31, checked on the host)
+        return p.k_cache + ((uint64_t)(uint32_t)sl[k] * (uint32_t)p.k_row_stride + co);
+      };
+      dma16_windows<0, C::NA - 1>(base, row_addr);
+      if (w < C::NAW) dma16_windows<C::NA - 1, C::NA>(base, row_addr);
+    } else {  // two caches: row waves, windows u = (w - RW0) + NRW k, K rows then V rows
+      if (w < C::RW0) return;
+      const uint32_t sbase = lds0 + st * C::STAGE;
+      // all slot reads first: each DMA below is an asm barrier for memory ops
+      int sl[C::NA], co[C::NA];
+#pragma unroll
+      for (int k = 0; k < C::NA; ++k) {
+        const int u = (w - C::RW0) + C::NRW * k;
+        if (u < C::KW) {
+          const int e = 64 * u + lane;  // 16-B chunk index within the stage
+          const int tok = e / C::KCPR, ch = e - tok * C::KCPR;
+          sl[k] = slot_of(t, ss, tok);
+          co[k] = 16 * min(ch, C::KCH - 1);
+        } else if (u < C::NW) {
+          const int e = 64 * (u - C::KW) + lane;
+          const int tok = e / C::VCPR, ch = e - tok * C::VCPR;
+          sl[k] = slot_of(t, ss, tok);
+          co[k] = 16 * min(ch, 31);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < C::NA; ++k) {
+        const int u = (w - C::RW0) + C::NRW * k;
+        if (u < C::KW)
+          dma16_to_lds_nt(p.k_cache + ((uint64_t)(uint32_t)sl[k] * (uint32_t)p.k_row_stride + (uint32_t)co[k]),
+                       sbase + 1024 * u);
+        else if (u < C::NW)
+          dma16_to_lds_nt(p.v_cache + ((uint64_t)(uint32_t)sl[k] * (uint32_t)p.v_row_stride + (uint32_t)co[k]),
+                       sbase + 1024 * u);
+      }
     }
   };
   // fp4 K scales: the 18 e8m0 bytes of token `lane` of tile t as 5 dwords
@@ -295,38 +347,41 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
   // 4, from byte 14: every read stays inside the row); dword j lands at
   // j * 64 + lane of the tile's scale stage.  A row starts at any byte (the
   // scale stride is free), so these are unaligned dword reads, which gfx950
-  // serves for global memory.  Columns j = w + SCW k are this wave's.
-  auto issue_scales = [&](int t) __attribute__((always_inline)) {
+  // serves for global memory.
+  auto issue_scales = [&](int t, int st, int ss) __attribute__((always_inline)) {
     if constexpr (KF == 1) {
-      if (w < C::SCW) {
-        const uint8_t* srow = p.k_scales + (uint64_t)(uint32_t)slot_of(t, lane) * (uint32_t)p.k_scale_stride;
-        const uint32_t sb = lds0 + C::OFF_SC + (t % C::S) * C::SCST;
+      const uint32_t sb = lds0 + C::OFF_SC + st * C::SCST;
+      if constexpr (C::VW == 0) {  // column w, and the last one on wave 3
+        const uint8_t* srow;
+        if (near_rows && kTile * (t + 1) <= ntok)
+          srow = p.k_scales + (int64_t)(t_beg + kTile * t) * p.k_scale_stride + (uint32_t)lane * (uint32_t)p.k_scale_stride;
+        else
+          srow = p.k_scales + (uint64_t)(uint32_t)slot_of(t, ss, lane) * (uint32_t)p.k_scale_stride;
+        dma4_to_lds(srow + 4 * w, sb + 256 * w);
+        if (w == 3) dma4_to_lds(srow + 14, sb + 256 * 4);
+      } else if (w == 0) {
+        const uint8_t* srow = p.k_scales + (uint64_t)(uint32_t)slot_of(t, ss, lane) * (uint32_t)p.k_scale_stride;
 #pragma unroll
-        for (int k = 0; k < (kScWin + C::SCW - 1) / C::SCW; ++k) {
-          const int j = w + C::SCW * k;
-          if (j < kScWin) dma4_to_lds(srow + (j < 4 ? 4 * j : 14), sb + 256 * j);
-        }
+        for (int j = 0; j < kScWin; ++j) dma4_to_lds(srow + (j < 4 ? 4 * j : 14), sb + 256 * j);
       }
     }
   };
   // this wave's wait for tile t's rows (and scales), k groups issued after them
   auto wait_tile = [&](int k) __attribute__((always_inline)) {
     constexpr int SL = IDX ? 1 : 0;  // wave 0 issues one slot DMA per group
-    if constexpr (KF == 1 && C::SCW == 4) {
-      // rows: NA for waves < NAW, else NA - 1; scale columns: 2 for wave 0, else 1
-      static_assert(C::RW0 == 0 && C::NAW == 3 && kScWin == 5, "per-wave DMA counts");
-      if (w == 0) wait_groups<C::NA + 2 + SL>(k);
-      else if (w == 1) wait_groups<C::NA + 1>(k);
-      else if (w == 2) wait_groups<C::NA + 1>(k);
-      else wait_groups<C::NA - 1 + 1>(k);
+    if constexpr (KF == 1 && C::VW == 0) {
+      // NA rows and one scale column, or NA - 1 rows and two (wave 3)
+      static_assert(C::NAW == 3 && kScWin == 5, "per-wave DMA counts");
+      if (IDX && w == 0) wait_groups<C::NA + 1 + SL>(k);
+      else wait_groups<C::NA + 1>(k);
     } else if constexpr (KF == 1) {
       // wave 0: one slot DMA + the 5 scale DMAs per group
       if (w == 0) wait_groups<kScWin + SL>(k);
       else if (w - C::RW0 < C::NAW) wait_groups<C::NA>(k);
       else wait_groups<C::NA - 1>(k);
     } else {
+      static_assert(C::NAW == 1, "only wave 0 has the last window");
       if (w == 0) wait_groups<C::NA + SL>(k);
-      else if (w < C::NAW) wait_groups<C::NA>(k);
       else wait_groups<C::NA - 1>(k);
     }
   };
@@ -339,7 +394,7 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
   // The first slot indices are in flight while Q is loaded (and quantized).
   if (ntiles > 0) {
 #pragma unroll
-    for (int j = 0; j < C::S; ++j) issue_slots(j);
+    for (int j = 0; j < C::S; ++j) issue_slots(j, j);
   }
 
   // ---- Q^T (B operand): head l16, dims 128ks + 32g .. +31 -------------------
@@ -530,12 +585,13 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
   float m_ref = 0.f, m_seen = neg_inf(), l_part = 0.f;
   bool have_ref = false;
   int e_ref = 127, e_seen = 0;  // fp4 V: reference and running max of the V block exponents
-  // (m_seen: fp8 V the wave's ceil max of a head, bf16 PV the lane's raw score max)
+  // (m_seen: fp8 V the wave's ceil max of a head, bf16 PV the lane's
+  // score max above m_ref)
 
   auto prologue = [&](bool slots_issued, bool quant) __attribute__((always_inline)) {
     if (!slots_issued) {
 #pragma unroll
-      for (int j = 0; j < C::S; ++j) issue_slots(j);
+      for (int j = 0; j < C::S; ++j) issue_slots(j, j);
     }
     wait_vmcnt<0>();
     lds_barrier();
@@ -543,9 +599,9 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
     for (int j = 0; j < C::S; ++j) {
       if (j >= ntiles) break;
       if (quant && j == C::S - 1) quantize_q();  // the other stages' rows are in flight
-      issue_slots(j + C::S);
-      issue_rows(j);
-      issue_scales(j);
+      issue_slots(j + C::S, j + C::S);
+      issue_rows(j, j, j);
+      issue_scales(j, j, j);
     }
     if (quant && ntiles < C::S) quantize_q();  // the last stage stays free
   };
@@ -553,11 +609,12 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
   // ---- main loop ---------------------------------------------------------------
   int8_t* vote = reinterpret_cast<int8_t*>(smem + C::OFF_VOTE);
   float* xch = reinterpret_cast<float*>(smem + C::OFF_X);
-  // bf16 PV: the item's references from the maxima seen so far (raw scores,
-  // V block exponents), over the lanes of a head and the waves
+  // bf16 PV: the item's references from the maxima seen so far (scores above
+  // the old reference, V block exponents), over the lanes of a head and the waves
   auto set_refs = [&]() __attribute__((always_inline)) {
     float mx = fmaxf(m_seen, shfl_xor_f(m_seen, 16));
-    mx = __builtin_ceilf(fmaxf(mx, shfl_xor_f(mx, 32)) * c);
+    mx = __builtin_ceilf(m_ref + fmaxf(mx, shfl_xor_f(mx, 32)));
+    m_seen = neg_inf();
     int* ex = reinterpret_cast<int*>(smem + C::OFF_E);
     const int e_w = C::VB16 ? wave_max(e_seen) : 0;
     if (g == 0) xch[16 * w + l16] = mx;
@@ -585,17 +642,20 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
     if (ntiles > 0) prologue(slots_issued, q_pending);
     slots_issued = false;
     q_pending = false;
-    for (int ti = 0; ti < ntiles; ++ti) {
-      const int st = ti % C::S;
+    // st = ti % S, ss = ti % NSL
+    for (int ti = 0, st = 0, ss = 0; ti < ntiles;
+         ++ti, st = st + 1 == C::S ? 0 : st + 1, ss = ss + 1 == C::NSL ? 0 : ss + 1) {
       const int nval = min(kTile, ntok - kTile * ti);
       // groups issued after group ti: 1 .. S-1 at the first tile, then the
       // S-2 before this pass's own issue
       wait_tile(min(ti == 0 ? C::S - 1 : C::S - 2, ntiles - 1 - ti));
       lds_barrier();  // (1) tile ti and its scales visible; iteration ti-1 done everywhere
       if (ti >= 1 && ti + C::S - 1 < ntiles) {
-        issue_slots(ti + 2 * C::S - 1);
-        issue_rows(ti + C::S - 1);
-        issue_scales(ti + C::S - 1);
+        const int si = st == 0 ? C::S - 1 : st - 1;  // stage of tile ti + S - 1, which tile ti - 1 used
+        const int sn = ss >= C::NSL - (C::S - 1) ? ss - (C::NSL - (C::S - 1)) : ss + C::S - 1;
+        issue_slots(ti + 2 * C::S - 1, ss == 0 ? C::NSL - 1 : ss - 1);
+        issue_rows(ti + C::S - 1, si, sn);
+        issue_scales(ti + C::S - 1, si, sn);
       }
       const uint8_t* kt = smem + st * C::STAGE;
       // e8m0 of (token t, block j): byte j & 3 of dword (j >> 2, t) at 256 (j >> 2)
@@ -649,8 +709,8 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
       if constexpr (C::PB) {
         // s[r] = score(token tok_of(w, 4g + r), head l16); positions past the
         // item repeat its last token, so they may enter the maxima
-        m_seen = fmaxf(fmaxf(m_seen, fmaxf(s[0], s[1])), fmaxf(s[2], s[3]));
         if (!have_ref) {  // first tile of the first pass
+          m_seen = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])) * c;
           set_refs();
           if constexpr (C::VB16) scale_steps(sct);
           have_ref = true;
@@ -659,7 +719,10 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
         // (fp4 V: with kVScaleSpan added to the exponent, see scale_steps)
         float pw[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) pw[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[r], c, -m_ref));
+        for (int r = 0; r < 4; ++r) pw[r] = __builtin_fmaf(s[r], c, -m_ref);
+        m_seen = fmaxf(fmaxf(m_seen, fmaxf(pw[0], pw[1])), fmaxf(pw[2], pw[3]));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) pw[r] = __builtin_amdgcn_exp2f(pw[r]);
         if (nval < kTile) {
 #pragma unroll
           for (int r = 0; r < 4; ++r) pw[r] = tok_of(w, 4 * g + r) < nval ? pw[r] : 0.f;
@@ -763,7 +826,8 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
         const int vst = VF == 1 ? C::VST : C::KST;
         const uint32_t vb = lds0 + st * C::STAGE + (VF == 1 ? C::KW * 1024 : 0) + 128 * w + 8 * (lane & 1);
         const int m = l16 >> 1;
-        const uint32_t a0 = vb + (16 * g0 + ih + m) * vst, a1 = vb + (16 * g1 + ih + m) * vst;
+        uint32_t a0 = vb + (16 * g0 + ih + m) * vst, a1 = vb + (16 * g1 + ih + m) * vst;
+        asm volatile("" : "+v"(a0), "+v"(a1));  // two addresses, the reads' offsets as immediates
         v2i r0[8], r1[8];
 #pragma unroll
         for (int dt = 0; dt < 8; ++dt) {
@@ -792,7 +856,8 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
         const uint4 p0 = *reinterpret_cast<const uint4*>(prow), p1 = *reinterpret_cast<const uint4*>(prow + 64);
         const uint32_t pq[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
         const int trow = l16 < 8 ? 8 * g + l16 : 24 + 8 * g + l16;
-        const uint32_t va = lds0 + st * C::STAGE + trow * C::KST + 64 * w;
+        uint32_t va = lds0 + st * C::STAGE + trow * C::KST + 64 * w;
+        asm volatile("" : "+v"(va));  // one address, the reads' offsets as immediates
         const uint8_t* et = smem + C::OFF_ET + 512 * w + 16 * g;
 #pragma unroll
         for (int jl = 0; jl < 4; ++jl) {  // block 4w + jl (dims 32(4w + jl) ..)
@@ -826,7 +891,7 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
     if constexpr (C::PB) {
       // a score or V block exponent too far above its reference anywhere in
       // the pass: run the item again from the maxima of the whole item
-      const bool over = ntiles > 0 && (__any(m_seen * c > m_ref + kRebase) ||
+      const bool over = ntiles > 0 && (__any(m_seen > kRebase) ||
                                        (C::VB16 && __any(e_seen > e_ref + kVScaleSpan)));
       if (lane == 0) vote[w] = over ? 1 : 0;
       lds_barrier();

@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 namespace mla {
 
 constexpr int kQKDim = 576;       // 512 latent + 64 rope
@@ -94,8 +96,8 @@ __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
 // two floats -> bf16 pair (RNE, v_cvt_pk_bf16_f32), a in the low half
 __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
-  const v2bf_t r = {(__bf16)a, (__bf16)b};
-  return __builtin_bit_cast(uint32_t, r);
+  typedef float v2f_t __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f_t{a, b}), v2bf_t));
 }
 
 // Round-to-nearest-even f32 -> OCP e4m3fn code for |f| <= 448.
@@ -271,6 +273,55 @@ __device__ __forceinline__ void dma2_to_lds(const void* g, uint32_t lds_off) { M
 // one byte per lane: lane l's byte lands, zero-extended, in the dword at M0 + 4 l
 __device__ __forceinline__ void dma1_to_lds(const void* g, uint32_t lds_off) { MLA_LDS_DMA("global_load_lds_ubyte %2, off"); }
 #undef MLA_LDS_DMA
+// A wave's DMA windows K0 .. K1 - 1 of a stage: window k lands at base + 4 KiB k
+// (base wave-uniform), lane l's 16 bytes from src(k) (a lane address), or from
+// the scalar address sb plus the lane offset src(k).  Four windows to an asm
+// block share one save and restore of M0; non-temporal as dma16_to_lds_nt.
+template <int I>
+using WinK = std::integral_constant<int, I>;
+#define MLA_WIN(OFF, SRC) \
+  "s_add_u32 m0, %1, " OFF "\n\ts_mov_b32 %0, %0\n\tglobal_load_lds_dwordx4 " SRC " nt\n\t"
+template <int K0, int K1, class F>
+__device__ __forceinline__ void dma16_windows(uint32_t base, F&& src) {
+  uint32_t saved;
+  if constexpr (K1 - K0 >= 4) {
+    asm volatile("s_mov_b32 %0, m0\n\t" MLA_WIN("%6", "%2, off") MLA_WIN("%7", "%3, off") MLA_WIN("%8", "%4, off")
+                     MLA_WIN("%9", "%5, off") "s_mov_b32 m0, %0"
+                 : "=&s"(saved)
+                 : "s"(base), "v"(src(WinK<K0>{})), "v"(src(WinK<K0 + 1>{})), "v"(src(WinK<K0 + 2>{})),
+                   "v"(src(WinK<K0 + 3>{})), "i"(4096 * K0), "i"(4096 * (K0 + 1)), "i"(4096 * (K0 + 2)),
+                   "i"(4096 * (K0 + 3))
+                 : "memory", "scc");
+    dma16_windows<K0 + 4, K1>(base, src);
+  } else if constexpr (K1 > K0) {
+    asm volatile("s_mov_b32 %0, m0\n\t" MLA_WIN("%3", "%2, off") "s_mov_b32 m0, %0"
+                 : "=&s"(saved)
+                 : "s"(base), "v"(src(WinK<K0>{})), "i"(4096 * K0)
+                 : "memory", "scc");
+    dma16_windows<K0 + 1, K1>(base, src);
+  }
+}
+template <int K0, int K1, class F>
+__device__ __forceinline__ void dma16_windows(uint32_t base, F&& src, const void* sb) {
+  uint32_t saved;
+  if constexpr (K1 - K0 >= 4) {
+    asm volatile("s_mov_b32 %0, m0\n\t" MLA_WIN("%7", "%2, %6") MLA_WIN("%8", "%3, %6") MLA_WIN("%9", "%4, %6")
+                     MLA_WIN("%10", "%5, %6") "s_mov_b32 m0, %0"
+                 : "=&s"(saved)
+                 : "s"(base), "v"(src(WinK<K0>{})), "v"(src(WinK<K0 + 1>{})), "v"(src(WinK<K0 + 2>{})),
+                   "v"(src(WinK<K0 + 3>{})), "s"(sb), "i"(4096 * K0), "i"(4096 * (K0 + 1)), "i"(4096 * (K0 + 2)),
+                   "i"(4096 * (K0 + 3))
+                 : "memory", "scc");
+    dma16_windows<K0 + 4, K1>(base, src, sb);
+  } else if constexpr (K1 > K0) {
+    asm volatile("s_mov_b32 %0, m0\n\t" MLA_WIN("%4", "%2, %3") "s_mov_b32 m0, %0"
+                 : "=&s"(saved)
+                 : "s"(base), "v"(src(WinK<K0>{})), "s"(sb), "i"(4096 * K0)
+                 : "memory", "scc");
+    dma16_windows<K0 + 1, K1>(base, src, sb);
+  }
+}
+#undef MLA_WIN
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
