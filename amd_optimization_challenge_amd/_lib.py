@@ -29,6 +29,7 @@ SIGNATURES = {
     "mla_abi_version": (_I, []),
     "mla_device_cu_count": (_I, [ctypes.POINTER(_I)]),
     "mla_workspace_bytes": (_I, [_I, _I, _I, ctypes.POINTER(_L)]),
+    "mla_workspace_bytes_qlen": (_I, [_I, _I, _I, _I, ctypes.POINTER(_L)]),
     "mla_quant_fp8_per_tensor": (_I, [_P, _L, _P, _P, _P, _L, _P]),
     "mla_pack_mxfp4": (_I, [_P, _L, _I, _L, _P, _L, _P, _L, _P]),
     "mla_append_kv": (_I, [_P, _L, _L, _P, _P, _L, _P, _P, _L, _P, _L, _P, _P]),
@@ -37,6 +38,7 @@ SIGNATURES = {
     "mla_decode": (_I, [_P, _P, _P, _L, _P, _L, _P, _L, _P, _P, _P, _I, _I, _F, _I, _P, _L, _P, _P, _P]),
     "mla_combine": (_I, [_I, _I, _P, _L, _P, _P, _P]),
     "mla_decode_fwd": (_I, [_P, _P, _L, _P, _L, _P, _L, _P, _P, _P, _I, _I, _I, _F, _I, _P, _L, _P, _P, _P]),
+    "mla_decode_fwd_rows": (_I, [_P, _P, _L, _P, _L, _P, _L, _P, _P, _P, _I, _I, _I, _F, _I, _P, _L, _P, _P, _P]),
     "mla_decode_fwd_a16w8": (_I, [_P, _P, _L, _P, _L, _P, _L, _P, _P, _P, _I, _I, _I, _F, _I, _P, _L, _P, _P, _P]),
     "mla_decode_fwd_rowq": (_I, [_P, _P, _L, _P, _L, _P, _L, _P, _P, _P, _I, _I, _I, _F, _I, _P, _L, _P, _P, _P]),
     "mla_absorb_q": (_I, [_P, _P, _P, _I, _I, _P, _P]),

@@ -144,6 +144,40 @@ WsLayout workspace_layout(int batch, int num_heads, int kv_mode, int num_cu) {
   return L;
 }
 
+// Causal rows of a sequence as one item (decode_rows.hip): `seqs` sequences of
+// qlen rows planned as sequences, one work-group per CU.  The partial outputs of
+// an item are qlen times a row's, so `cap` items fit the workspace given: all of
+// plan_target_for's where the workspace is sized by mla_workspace_bytes_qlen,
+// fewer (at least seqs + 127 of the CUs' 256) in one sized by
+// mla_workspace_bytes.
+struct RowsLayout {
+  PlanTarget target;
+  int grid;  // most items the planner emits
+  int64_t part_lse_off;
+};
+static int64_t rows_part_bytes(int64_t items, int cols) {
+  return align256(items * cols * kVDim * 2) + align256(items * cols * 4);
+}
+static RowsLayout rows_layout(const WsLayout& L, int seqs, int qlen, int num_cu, bool contiguous, int64_t workspace_bytes) {
+  const int cols = 16 * qlen;
+  RowsLayout R;
+  // target_items_for's rule at one resident work-group per CU (as for 128 heads)
+  R.target = PlanTarget{target_items_for(seqs, 128, MLA_KV_FP8, num_cu), kPlanMinChunk, contiguous ? 32 : 0};
+  int64_t cap = (workspace_bytes - L.part_o_off - 512) / ((int64_t)cols * (kVDim * 2 + 4));
+  if (cap > L.max_items) cap = L.max_items;  // the plan's room
+  // up to 256 rows the planner keeps within max(target, seqs) items, past that
+  // within target + seqs
+  const int64_t most = seqs <= 256 ? cap : cap - seqs;
+  if (R.target.items > most) R.target.items = (int)most;
+  R.grid = seqs <= 256 ? (R.target.items > seqs ? R.target.items : seqs) : R.target.items + seqs;
+  R.part_lse_off = L.part_o_off + align256((int64_t)R.grid * cols * kVDim * 2);
+  return R;
+}
+// what decode_rows.hip takes
+static bool rows_as_one_item(int q_seq_len, int num_heads, int kv_mode) {
+  return num_heads == 16 && kv_mode == MLA_KV_FP8 && q_seq_len >= 2 && q_seq_len <= kMaxRowsPerItem;
+}
+
 namespace {
 
 int decode_params(const void* q_fp8, const float* q_scale, const void* k_cache, int64_t k_row_stride,
@@ -242,6 +276,21 @@ int mla_workspace_bytes(int batch, int num_heads, int kv_mode, int64_t* bytes) {
   int ncu = 0;
   if ((rc = cu_count(&ncu))) return rc;
   *bytes = workspace_layout(batch, num_heads, kv_mode, ncu).total;
+  return MLA_OK;
+}
+
+int mla_workspace_bytes_qlen(int batch, int q_seq_len, int num_heads, int kv_mode, int64_t* bytes) {
+  int rc = mla_workspace_bytes(batch, num_heads, kv_mode, bytes);
+  if (rc) return rc;
+  if ((rc = check_qlen(batch, q_seq_len))) return rc;
+  if (rows_as_one_item(q_seq_len, num_heads, kv_mode)) {
+    int ncu = 0;
+    if ((rc = cu_count(&ncu))) return rc;
+    const WsLayout L = workspace_layout(batch, num_heads, kv_mode, ncu);
+    const RowsLayout R = rows_layout(L, batch / q_seq_len, q_seq_len, ncu, false, INT64_MAX / 2);
+    const int64_t need = L.part_o_off + 512 + rows_part_bytes(R.grid, 16 * q_seq_len);
+    if (need > *bytes) *bytes = need;
+  }
   return MLA_OK;
 }
 
@@ -458,6 +507,52 @@ int mla_decode_fwd(const void* q_bf16, const void* k_cache, int64_t k_row_stride
     if (e != hipSuccess) return hip_fail(e, "quant launch");
   }
   e = launch_decode(p, kv_mode, L.max_items, s);
+  if (e != hipSuccess) return hip_fail(e, "decode launch");
+  e = launch_combine(p, s);
+  if (e != hipSuccess) return hip_fail(e, "combine launch");
+  return MLA_OK;
+}
+
+int mla_decode_fwd_rows(const void* q_bf16, const void* k_cache, int64_t k_row_stride, const void* k_scales,
+                        int64_t k_scale_stride, const void* v_cache, int64_t v_row_stride,
+                        const float* kv_scale, const int32_t* kv_indptr, const int32_t* kv_indices, int batch,
+                        int q_seq_len, int num_heads, float sm_scale, int kv_mode, void* workspace,
+                        int64_t workspace_bytes, void* out_bf16, float* lse_out, void* stream) {
+  if (!rows_as_one_item(q_seq_len, num_heads, kv_mode))
+    return set_error(MLA_ERR_UNSUPPORTED,
+                     "rows as one item: 16 heads, the fp8 cache and q_seq_len 2 to %d (got %d, kv_mode %d, %d)",
+                     kMaxRowsPerItem, num_heads, kv_mode, q_seq_len);
+  if (!q_bf16 || !aligned(q_bf16, 16)) return set_error(MLA_ERR_INVALID_ARGUMENT, "q must be non-null and 16-byte aligned");
+  int rc = check_shape(batch, num_heads, kv_mode);
+  if (rc) return rc;
+  if ((rc = check_qlen(batch, q_seq_len))) return rc;
+  int ncu = 0;
+  if ((rc = cu_count(&ncu))) return rc;
+  DecodeParams p{};
+  WsLayout L = workspace_layout(batch, num_heads, kv_mode, ncu);
+  char* ws = static_cast<char*>(workspace);
+  // the fp8 Q slots of the workspace are not read on this route
+  rc = decode_params(q_bf16, reinterpret_cast<const float*>(ws + L.quant_off + 4096), k_cache, k_row_stride, k_scales,
+                     k_scale_stride, v_cache, v_row_stride, kv_scale, kv_indptr, kv_indices, batch, num_heads, sm_scale,
+                     kv_mode, workspace, workspace_bytes, out_bf16, lse_out, &p, &L);
+  if (rc) return rc;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const int seqs = batch / q_seq_len;
+  const RowsLayout R = rows_layout(L, seqs, q_seq_len, ncu, kv_indices == nullptr, workspace_bytes);
+  uint32_t* partials = reinterpret_cast<uint32_t*>(ws + L.quant_off);
+  int nb = 0;
+  hipError_t e = launch_amax(static_cast<const uint16_t*>(q_bf16), (int64_t)batch * num_heads * kQKDim, partials, &nb,
+                             kv_indptr, kv_indices, seqs, 1, R.target, L.max_items,
+                             reinterpret_cast<int32_t*>(ws + L.plan_off), s);
+  if (e != hipSuccess) return hip_fail(e, "amax+plan launch");
+  p.q_bf16 = static_cast<const uint16_t*>(q_bf16);
+  p.q_partials = partials;
+  p.q_nparts = nb;
+  p.part_lse = reinterpret_cast<float*>(ws + R.part_lse_off);
+  p.batch = seqs;
+  p.num_heads = num_heads * q_seq_len;
+  p.plan_qlen = q_seq_len;
+  e = launch_decode_rows(p, R.grid, s);
   if (e != hipSuccess) return hip_fail(e, "decode launch");
   e = launch_combine(p, s);
   if (e != hipSuccess) return hip_fail(e, "combine launch");

@@ -72,6 +72,7 @@
 #include <type_traits>
 
 #include "mla_internal.hpp"
+#include "mla_tile64.hpp"
 
 namespace mla {
 namespace {
@@ -81,7 +82,7 @@ constexpr float kLn2F = 0.6931471805599453f;
 constexpr float kRebaseF = 96.0f;
 
 struct G128 {
-  static constexpr int RST = 608;               // LDS row stride
+  static constexpr int RST = kRowSt;            // LDS row stride
   static constexpr int CPR = RST / 16;          // 38 chunk positions per row (36 used)
   static constexpr int HT = 32;                 // tokens per tile
   static constexpr int TSTAGE = HT * RST;       // 19456 B per tile
@@ -120,13 +121,6 @@ struct M128 {
   static_assert(OFF_Q + 128 * kQKDim <= OFF_S, "Q staging stays clear of the e8m0 stages");
   static_assert(LDS <= 160 * 1024, "LDS");
 };
-
-__device__ __forceinline__ int g128_key(int r) { return (r >> 2) & 7; }
-// LDS chunk position (0..35) of logical chunk c of row r; an involution
-__device__ __forceinline__ int g128_pos(int r, int c) {
-  const int x = g128_key(r);
-  return c < 32 ? (c ^ x) : 32 + ((c - 32) ^ (x & 3));
-}
 
 __device__ __forceinline__ float ninf() { return -__builtin_inff(); }
 
@@ -185,16 +179,6 @@ __device__ __forceinline__ void pv_mfma(v16f& acc, const v8i& a, const v8i& b, i
                : "+a"(acc)
                : "v"(a), "v"(b), "v"(127), "v"(bscale));
 }
-// v_permlane32_swap of x with itself: each lane ends with its own value and
-// its partner's (lane +- 32)
-__device__ __forceinline__ float xhalf_max(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float xhalf_sum(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
 // max of three scores (no NaN canonicalization: the scores are MFMA outputs)
 __device__ __forceinline__ float max3f(float a, float b, float c) {
   float r;
@@ -210,14 +194,6 @@ __device__ __forceinline__ float mask_ge(float x, int pos, int lim) {
       : "vcc");
   return x;
 }
-// {hi, lo}: hi = e4m3(x), lo = e4m3(x - hi) of four values in [0, 448)
-__device__ __forceinline__ int2 split4(float a, float b, float c, float d) {
-  const uint32_t h = pack4_fp8(a, b, c, d);
-  const v2f h01 = __builtin_amdgcn_cvt_pk_f32_fp8((int)h, false);
-  const v2f h23 = __builtin_amdgcn_cvt_pk_f32_fp8((int)h, true);
-  return make_int2((int)h, (int)pack4_fp8(a - h01[0], b - h01[1], c - h23[0], d - h23[1]));
-}
-
 template <int I>
 using Ic = std::integral_constant<int, I>;
 

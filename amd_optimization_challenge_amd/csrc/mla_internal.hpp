@@ -77,6 +77,11 @@ hipError_t launch_combine(const DecodeParams& p, hipStream_t stream);
 hipError_t launch_decode_h128f(const DecodeParams& p, int grid, hipStream_t stream);
 hipError_t launch_decode_h128m(const DecodeParams& p, int grid, hipStream_t stream);
 
+// decode_rows.hip: 16 heads, fp8 cache, the p.plan_qlen (2 .. kMaxRowsPerItem)
+// causal rows of a sequence as one item of 16 plan_qlen heads
+constexpr int kMaxRowsPerItem = 4;
+hipError_t launch_decode_rows(const DecodeParams& p, int grid, hipStream_t stream);
+
 // neighbours.hip
 hipError_t launch_absorb_q(const uint16_t* q_nope, const uint16_t* q_rope, const uint16_t* w_uk, int batch,
                            int heads, uint16_t* q_out, hipStream_t stream);

@@ -54,24 +54,25 @@ def cu_count() -> int:
     return n.value
 
 
-def workspace_bytes(batch: int, num_heads: int, kv_mode) -> int:
+def workspace_bytes(batch: int, num_heads: int, kv_mode, q_seq_len: int = 1) -> int:
     n = ctypes.c_int64(0)
-    _lib.check(_lib.load().mla_workspace_bytes(batch, num_heads, kv_mode_id(kv_mode), ctypes.byref(n)),
-               "mla_workspace_bytes")
+    _lib.check(_lib.load().mla_workspace_bytes_qlen(batch, q_seq_len, num_heads, kv_mode_id(kv_mode),
+                                                    ctypes.byref(n)),
+               "mla_workspace_bytes_qlen")
     return n.value
 
 
 _ws_cache: dict = {}
 
 
-def workspace(batch: int, num_heads: int, kv_mode, device) -> torch.Tensor:
+def workspace(batch: int, num_heads: int, kv_mode, device, q_seq_len: int = 1) -> torch.Tensor:
     """Workspace for a shape, cached per (shape, device) -- keyed on shapes only."""
     device = torch.device(device)
-    key = (batch, num_heads, kv_mode_id(kv_mode), device)
+    key = (batch, num_heads, kv_mode_id(kv_mode), device, q_seq_len)
     ws = _ws_cache.get(key)
     if ws is None:
         with torch.cuda.device(device):
-            ws = torch.empty(workspace_bytes(batch, num_heads, kv_mode), dtype=torch.uint8, device=device)
+            ws = torch.empty(workspace_bytes(batch, num_heads, kv_mode, q_seq_len), dtype=torch.uint8, device=device)
         _ws_cache[key] = ws
     return ws
 
@@ -266,6 +267,19 @@ def combine(batch: int, num_heads: int, ws: torch.Tensor, out: torch.Tensor, lse
                                            _stream()), "mla_combine")
 
 
+def _rows_together(q_seq_len: int, num_heads: int, mode: int, tokens: int) -> bool:
+    """The causal rows of a sequence as one pass over its cache
+    (``mla_decode_fwd_rows``) instead of a pass per row.  It saves q_seq_len - 1
+    gathers of at most ``tokens`` cached rows (580 bytes at about 5.4 TB/s) and
+    costs about 4 us of longer prologue and finish per work-group (64 columns,
+    one work-group per CU), so it pays from (q_seq_len - 1) x tokens = 2^15.
+    Whole calls on MI355X, a pass per row against this: 60 x 160 tokens x 4 rows
+    19.7 / 23.7 us and 32 x 800 x 2 22.9 / 23.3 (below the line), 100 x 200 x 3
+    31.6 / 25.9, 300 x 40 x 4 38.2 / 34.1 and 32 of 512 to 8192 x 4 58.0 / 33.3
+    (above it)."""
+    return num_heads == 16 and mode == 0 and 2 <= q_seq_len <= 4 and (q_seq_len - 1) * tokens >= 1 << 15
+
+
 def decode_fwd(q, kv_data, kv_indptr, kv_indices, sm_scale, kv_mode="fp8", out=None, ws=None, q_seq_len=1,
                return_lse=False, page_size=1, kv_last_page_lens=None, q_dtype="fp8", lse=None):
     """Whole operator: FP8-quantize q, plan, decode, combine.
@@ -280,7 +294,9 @@ def decode_fwd(q, kv_data, kv_indptr, kv_indices, sm_scale, kv_mode="fp8", out=N
     cache): Q keeps its own precision, no per-tensor quantization.  q_dtype
     "fp8_row" (``mla_decode_fwd_rowq``; 16 heads, fp8 or mxfp4 cache): Q
     quantized per head row inside the decode, which for up to 256 query rows
-    also plans its own work (two launches per call).  ``out`` (bf16 [rows, H,
+    also plans its own work (two launches per call).  q_dtype "fp8" with 16
+    heads, the fp8 cache, q_seq_len 2 to 4 and enough cached tokens runs a
+    sequence's rows together (``_rows_together``).  ``out`` (bf16 [rows, H,
     512]) and ``lse`` (f32 [rows, H], with ``return_lse``) may be passed in;
     each is allocated here only when it is not.
     """
@@ -301,8 +317,10 @@ def decode_fwd(q, kv_data, kv_indptr, kv_indices, sm_scale, kv_mode="fp8", out=N
                          f"entries do not fit (need rows = sequences x q_seq_len, indptr = sequences + 1)")
     mode = kv_mode_id(kv_mode)
     k, ks, ksc, kss, v, vs, sc = _kv_args(mode, kv_data)
+    rows = q_dtype == "fp8" and _rows_together(q_seq_len, num_heads, mode,
+                                               k.shape[0] if kv_indices is None else kv_indices.numel())
     if ws is None:
-        ws = workspace(batch, num_heads, mode, q.device)
+        ws = workspace(batch, num_heads, mode, q.device, q_seq_len if rows else 1)
     if out is None:
         out = torch.empty((batch, num_heads, V_DIM), dtype=torch.bfloat16, device=q.device)
     elif out.dtype != torch.bfloat16 or tuple(out.shape) != (batch, num_heads, V_DIM) or not out.is_contiguous():
@@ -317,7 +335,7 @@ def decode_fwd(q, kv_data, kv_indptr, kv_indices, sm_scale, kv_mode="fp8", out=N
     if q_dtype not in routes:
         raise ValueError(f"q_dtype must be 'fp8' (a8w8: per-tensor Q quant), 'bf16' (a16w8) or 'fp8_row' "
                          f"(per-row Q quant), got {q_dtype!r}")
-    name = routes[q_dtype]
+    name = "mla_decode_fwd_rows" if rows else routes[q_dtype]
     fn = getattr(_lib.load(), name)
     with torch.cuda.device(q.device):
         _lib.check(fn(

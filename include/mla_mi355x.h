@@ -70,6 +70,14 @@ int mla_device_cu_count(int* num_cu);
 int mla_workspace_bytes(int batch, int num_heads, int kv_mode, int64_t* bytes);
 
 /*
+ * The same for a call of `batch` query rows, q_seq_len per sequence.  Never less
+ * than mla_workspace_bytes, which every entry point accepts; with 16 heads, the
+ * fp8 cache and q_seq_len 2 to 4 (mla_decode_fwd_rows) it holds the partial outputs of a piece per compute unit
+ * (a smaller workspace means fewer, longer pieces).
+ */
+int mla_workspace_bytes_qlen(int batch, int q_seq_len, int num_heads, int kv_mode, int64_t* bytes);
+
+/*
  * Per-tensor FP8 quantization of n bf16 values: amax -> scale = bf16(amax/448)
  * -> e4m3fn(clamp(bf16(x/scale), +-448)), bit-exact to quantize_fp8
  * (competitor_submissions/mi355x_reference/reference.py:65-80).  Writes the f32
@@ -202,6 +210,19 @@ int mla_decode_fwd(const void* q_bf16, const void* k_cache, int64_t k_row_stride
                    const int32_t* kv_indptr, const int32_t* kv_indices, int batch,
                    int q_seq_len, int num_heads, float sm_scale, int kv_mode, void* workspace,
                    int64_t workspace_bytes, void* out_bf16, float* lse_out, void* stream);
+
+/*
+ * mla_decode_fwd for the causal rows of multi-token sequences (16 heads, fp8
+ * cache, q_seq_len 2 to 4): the rows of a sequence share one pass over its
+ * cache instead of a pass each.  Same arguments and result; it pays once
+ * (q_seq_len - 1) x cached tokens is above about 32768 (ops.decode_fwd's rule).
+ * Workspace: mla_workspace_bytes_qlen, or at least mla_workspace_bytes.
+ */
+int mla_decode_fwd_rows(const void* q_bf16, const void* k_cache, int64_t k_row_stride, const void* k_scales,
+                        int64_t k_scale_stride, const void* v_cache, int64_t v_row_stride,
+                        const float* kv_scale, const int32_t* kv_indptr, const int32_t* kv_indices, int batch,
+                        int q_seq_len, int num_heads, float sm_scale, int kv_mode, void* workspace,
+                        int64_t workspace_bytes, void* out_bf16, float* lse_out, void* stream);
 
 /*
  * The a16w8 route: bf16 Q against the fp8 cache with no tensor-wide Q scale,

@@ -1,0 +1,106 @@
+"""The causal rows of a sequence as one work item (16 heads, fp8 cache, q_seq_len 2
+to 4) at the edges of its tiles: one-token to many-tile sequences, rows that see
+nothing, pieces whose end lies inside the last rows' masked tail, a second pass from
+higher references, more sequences than the planner sorts, and workspaces of both
+sizes; against the oracle."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from amd_optimization_challenge_amd import _lib, ops
+from mla_cases import assert_close, case_from_tensors, device_data, host_case
+from oracle import mla_oracle as O
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+
+
+@pytest.fixture(autouse=True)
+def _rows_route(monkeypatch):
+    """Every test here takes the route, whatever its size."""
+    rule = ops._rows_together
+    monkeypatch.setattr(ops, "_rows_together", lambda n, h, mode, tokens: rule(n, h, mode, 1 << 30))
+
+
+def _run(case, q, qlen, sm, contiguous=False, ws=None):
+    _, kv, indptr, idx, _, caches = case
+    S = indptr.numel() - 1
+    _, kv_data, _, kv_indptr, cfg = device_data(q[:S], kv, indptr, idx, caches, "fp8", sm, pass_indices=not contiguous)
+    return ops.decode_fwd(q.to(DEV), kv_data, kv_indptr, cfg["kv_indices"], sm, "fp8", ws=ws, q_seq_len=qlen,
+                          return_lse=True)
+
+
+def _check(case, q, qlen, sm, out, lse):
+    _, _, indptr, idx, _, caches = case
+    _, ref, ref_lse = O.reference_path(O.bf16_tensor_bits(q), "fp8", caches, indptr.numpy(), idx.numpy(), sm,
+                                       q_seq_len=qlen, return_lse=True)
+    assert_close(out.float().cpu().numpy(), ref)
+    got = lse.cpu().numpy()
+    assert np.array_equal(np.isneginf(got), np.isneginf(ref_lse))
+    fin = ~np.isneginf(ref_lse)
+    # an lse error d scales the row's weights by e^d: 1e-2 stays inside the 2e-2 of the output
+    assert np.all(np.abs(got[fin] - ref_lse[fin]) <= 1e-2 + 1e-2 * np.abs(ref_lse[fin]))
+
+
+@pytest.mark.parametrize("qlen", [2, 3, 4])
+@pytest.mark.parametrize("contiguous", [False, True])
+@pytest.mark.parametrize("lens", [[1], [3, 2, 64], [63, 65, 66], [130, 0, 127, 129], [2049], [191] * 40])
+def test_rows_match_oracle(qlen, contiguous, lens):
+    g = torch.Generator().manual_seed(sum(lens) + qlen)
+    q = torch.randn(len(lens) * qlen, 16, 576, generator=g).to(torch.bfloat16)
+    case = host_case(lens, 16, "fp8", seed=3 + qlen, permute=not contiguous)
+    out, lse = _run(case, q, qlen, 0.08, contiguous)
+    _check(case, q, qlen, 0.08, out, lse)
+
+
+def test_more_sequences_than_the_planner_sorts():
+    lens = [(7 * i) % 90 for i in range(300)]
+    q = torch.randn(600, 16, 576, generator=torch.Generator().manual_seed(1)).to(torch.bfloat16)
+    case = host_case(lens, 16, "fp8", seed=9)
+    out, lse = _run(case, q, 2, 0.08)
+    _check(case, q, 2, 0.08, out, lse)
+
+
+def test_second_pass_from_higher_references():
+    """Scores that climb by ~100 (log2 units) per tile: past the accumulators' range."""
+    g = torch.Generator().manual_seed(17)
+    lens, qlen = [700, 130, 5], 4
+    T = sum(lens)
+    q = torch.randn(len(lens) * qlen, 16, 576, generator=g)
+    q[..., 7] = 40.0
+    kv = 0.25 * torch.randn(T, 1, 576, generator=g)
+    pos = torch.cat([torch.arange(L) for L in lens]).float()
+    kv[:, 0, 7] = 6.0 * torch.floor(pos / 64) - 20.0 + 0.1 * torch.randn(T, generator=g)
+    indptr = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32)
+    idx = torch.randperm(T, generator=g).to(torch.int32)
+    rows = torch.empty_like(kv)
+    rows[idx.long()] = kv
+    case = case_from_tensors(q[:3].to(torch.bfloat16), rows.to(torch.bfloat16), indptr, idx, "fp8")
+    qb = q.to(torch.bfloat16)
+    out, lse = _run(case, qb, qlen, 1 / np.sqrt(192))
+    assert torch.isfinite(out).all()
+    _check(case, qb, qlen, 1 / np.sqrt(192), out, lse)
+
+
+@pytest.mark.parametrize("qlen", [2, 4])
+def test_workspace_sizes(qlen):
+    """The size of mla_workspace_bytes is accepted (fewer pieces), a byte less refused."""
+    lens = [3000, 900, 40]
+    q = torch.randn(3 * qlen, 16, 576, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16)
+    case = host_case(lens, 16, "fp8", seed=4)
+    n = ctypes.c_int64(0)
+    _lib.check(_lib.load().mla_workspace_bytes(3 * qlen, 16, 0, ctypes.byref(n)), "mla_workspace_bytes")
+    assert ops.workspace_bytes(3 * qlen, 16, "fp8", qlen) >= n.value == ops.workspace_bytes(3 * qlen, 16, "fp8")
+    ws = torch.empty(n.value, dtype=torch.uint8, device=DEV)
+    out, lse = _run(case, q, qlen, 0.08, ws=ws)
+    _check(case, q, qlen, 0.08, out, lse)
+    with pytest.raises(_lib.MlaLibraryError):
+        _run(case, q, qlen, 0.08, ws=ws[:-256])
+
+
+def test_route_rule():
+    """The line of the dispatch (undisturbed by the fixture's size)."""
+    assert ops._rows_together(4, 16, 0, 0) and ops._rows_together(2, 16, 0, 0)
+    assert not any(ops._rows_together(*a, 0) for a in [(1, 16, 0), (5, 16, 0), (4, 128, 0), (4, 16, 1), (4, 16, 3)])
