@@ -62,6 +62,8 @@ _lib = None
 def load(path: str = LIB_PATH) -> ctypes.CDLL:
     """Load (once) and return the library with all signatures bound."""
     global _lib
+    if _lib is not None:
+        return _lib
     with _lock:
         if _lib is not None:
             return _lib

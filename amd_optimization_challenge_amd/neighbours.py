@@ -21,8 +21,7 @@ from __future__ import annotations
 
 import torch
 
-from . import _lib
-from .ops import _ptr, _stream
+from .ops import _call, _ptr
 
 QK_NOPE = 128   # DeepSeek-V3/R1 qk_nope_head_dim
 QK_ROPE = 64    # qk_rope_head_dim
@@ -50,9 +49,7 @@ def absorb_q(q_nope: torch.Tensor, q_rope: torch.Tensor, w_uk: torch.Tensor) -> 
            (w_uk, "w_uk", (H, QK_NOPE, LATENT)))
     q_nope, q_rope, w_uk = q_nope.contiguous(), q_rope.contiguous(), w_uk.contiguous()
     out = torch.empty((B, H, LATENT + QK_ROPE), dtype=torch.bfloat16, device=q_nope.device)
-    with torch.cuda.device(q_nope.device):
-        _lib.check(_lib.load().mla_absorb_q(_ptr(q_nope), _ptr(q_rope), _ptr(w_uk), B, H, _ptr(out),
-                                            _stream()), "mla_absorb_q")
+    _call("mla_absorb_q", q_nope.device, _ptr(q_nope), _ptr(q_rope), _ptr(w_uk), B, H, _ptr(out))
     return out
 
 
@@ -69,8 +66,6 @@ def v_up_proj(o: torch.Tensor, w_uv: torch.Tensor, quant_fp8: bool = False):
         q8 = torch.empty((B, H, V_HEAD), dtype=torch.float8_e4m3fn, device=o.device)
         scale = torch.empty(1, dtype=torch.float32, device=o.device)
         scratch = torch.empty(8192, dtype=torch.uint8, device=o.device)
-    with torch.cuda.device(o.device):
-        _lib.check(_lib.load().mla_v_up_proj(_ptr(o), _ptr(w_uv), B, H, _ptr(y), _ptr(q8), _ptr(scale),
-                                             _ptr(scratch), 0 if scratch is None else scratch.numel(),
-                                             _stream()), "mla_v_up_proj")
+    _call("mla_v_up_proj", o.device, _ptr(o), _ptr(w_uv), B, H, _ptr(y), _ptr(q8), _ptr(scale), _ptr(scratch),
+          0 if scratch is None else scratch.numel())
     return (q8, scale) if quant_fp8 else y
