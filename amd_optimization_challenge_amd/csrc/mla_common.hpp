@@ -81,6 +81,12 @@ __device__ __forceinline__ uint4 ldg16_nt(const void* p) {
   return make_uint4(v[0], v[1], v[2], v[3]);
 }
 
+// 8-byte streaming store (written once; not read soon)
+__device__ __forceinline__ void stg8_nt(uint2* p, uint2 v) {
+  typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+  __builtin_nontemporal_store((u32x2{v.x, v.y}), reinterpret_cast<u32x2*>(p));
+}
+
 // ---- bf16 / fp8 scalar conversions (bit exact, no fast math) ----------------
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t h) {
   return __uint_as_float(h << 16);
