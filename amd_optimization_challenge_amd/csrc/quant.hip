@@ -229,6 +229,7 @@ __global__ __launch_bounds__(256) void pack_mxfp4_kernel(const uint8_t* __restri
 // skipped or written, so the 4 lanes of a block are active together.
 // ---------------------------------------------------------------------------
 constexpr int kLanesPerToken = kQKDim / 8;  // 72
+constexpr uint32_t kAppendUnroll = 2;  // chunks in flight per lane (65536 tokens: 33.3 us at 1, 31.6 at 2, 33.4 at 4)
 
 __global__ __launch_bounds__(256) void append_kv_kernel(
     const uint8_t* __restrict__ x, int n, int64_t x_stride, const int32_t* __restrict__ slots,
@@ -238,26 +239,43 @@ __global__ __launch_bounds__(256) void append_kv_kernel(
   const uint32_t total = (uint32_t)n * kLanesPerToken;
   const Fp8Quant s = make_fp8_quant(fp8_cache != nullptr ? fp8_scale[0] : 1.0f);
   uint32_t amax = 0;  // bf16 |x| bits over this lane's written chunks
-  for (uint32_t u = blockIdx.x * 256u + threadIdx.x; u < total; u += gridDim.x * 256u) {
-    const uint32_t t = u / kLanesPerToken;
-    const uint32_t p = u - t * kLanesPerToken;
-    const int64_t slot = slots != nullptr ? (int64_t)slots[t] : (int64_t)t;
-    if (slot < 0) continue;
-    const uint4 v = ldg16_nt(x + (int64_t)t * x_stride + p * 16);
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-    uint32_t m = 0;
+  const uint32_t step = gridDim.x * 256u;
+  for (uint32_t u0 = blockIdx.x * 256u + threadIdx.x; u0 < total; u0 += kAppendUnroll * step) {
+    // the slots and values of kAppendUnroll chunks are in flight together (a
+    // skipped token's values are read and dropped)
+    uint4 vv[kAppendUnroll];
+    int sl[kAppendUnroll];
 #pragma unroll
-    for (int k = 0; k < 4; ++k) m = max(m, max(w[k] & 0x7FFFu, (w[k] >> 16) & 0x7FFFu));
-    amax = max(amax, m);
-    if (fp8_cache != nullptr)
-      *reinterpret_cast<uint2*>(fp8_cache + slot * fp8_stride + p * 8) = quant8_fp8(v, s);
-    if (fp4_cache != nullptr) {
-      m = max(m, (uint32_t)__shfl_xor((int)m, 1, 64));
-      m = max(m, (uint32_t)__shfl_xor((int)m, 2, 64));
-      const int e = mx_exponent(m << 16);
-      const float qs = mx_qscale(e);
-      *reinterpret_cast<uint32_t*>(fp4_cache + slot * fp4_stride + p * 4) = mx_encode_word4(w[0], w[1], w[2], w[3], qs);
-      if ((p & 3u) == 0) fp4_scales[slot * fp4_scale_stride + (p >> 2)] = (uint8_t)(e + 127);
+    for (uint32_t k = 0; k < kAppendUnroll; ++k) {
+      const uint32_t u = u0 + k * step;
+      sl[k] = -1;
+      if (u0 < total - k * step && k * step < total) {  // u < total, without overflow
+        const uint32_t t = u / kLanesPerToken;
+        vv[k] = ldg16_nt(x + (int64_t)t * x_stride + (u - t * kLanesPerToken) * 16);
+        sl[k] = slots != nullptr ? slots[t] : (int)t;
+      }
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < kAppendUnroll; ++k) {
+      if (sl[k] < 0) continue;
+      const uint32_t u = u0 + k * step;
+      const uint32_t p = u % kLanesPerToken;
+      const int64_t slot = sl[k];
+      const uint32_t w[4] = {vv[k].x, vv[k].y, vv[k].z, vv[k].w};
+      uint32_t m = 0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) m = max(m, max(w[e] & 0x7FFFu, (w[e] >> 16) & 0x7FFFu));
+      amax = max(amax, m);
+      if (fp8_cache != nullptr)
+        *reinterpret_cast<uint2*>(fp8_cache + slot * fp8_stride + p * 8) = quant8_fp8(vv[k], s);
+      if (fp4_cache != nullptr) {
+        m = max(m, (uint32_t)__shfl_xor((int)m, 1, 64));
+        m = max(m, (uint32_t)__shfl_xor((int)m, 2, 64));
+        const int e = mx_exponent(m << 16);
+        const float qs = mx_qscale(e);
+        *reinterpret_cast<uint32_t*>(fp4_cache + slot * fp4_stride + p * 4) = mx_encode_word4(w[0], w[1], w[2], w[3], qs);
+        if ((p & 3u) == 0) fp4_scales[slot * fp4_scale_stride + (p >> 2)] = (uint8_t)(e + 127);
+      }
     }
   }
   if (amax_out != nullptr) {
