@@ -492,6 +492,21 @@ int mla_decode_fwd(const void* q_bf16, const void* k_cache, int64_t k_row_stride
     if (e != hipSuccess) return hip_fail(e, "combine launch");
     return MLA_OK;
   }
+  if (num_heads == 16 && batch <= kSelfAmaxRows && (kv_mode == MLA_KV_FP8 || kv_mode == MLA_KV_MXFP4)) {
+    // the decode plans its own work and scales its own Q: one launch fewer
+    const PlanTarget t = plan_target_for(batch, num_heads, kv_mode, ncu, kv_indices == nullptr);
+    p.q_bf16 = static_cast<const uint16_t*>(q_bf16);
+    p.plan_here = 1;
+    p.plan_qlen = q_seq_len;
+    p.plan_target = t.items;
+    p.plan_min_chunk = t.min_chunk;
+    p.plan_max_splits = t.max_splits;
+    hipError_t e = launch_decode(p, kv_mode, t.items + batch < L.max_items ? t.items + batch : L.max_items, s);
+    if (e != hipSuccess) return hip_fail(e, "decode launch");
+    e = launch_combine(p, s);
+    if (e != hipSuccess) return hip_fail(e, "combine launch");
+    return MLA_OK;
+  }
   hipError_t e = launch_amax(static_cast<const uint16_t*>(q_bf16), n, partials, &nb, kv_indptr,
                              static_cast<const int32_t*>(kv_indices), batch, q_seq_len,
                              plan_target_for(batch, num_heads, kv_mode, ncu, kv_indices == nullptr),

@@ -174,7 +174,9 @@ constexpr int kVScaleSpan = 31;  // fp4 V: P' = P 2^(e - E_ref) <= 2^(96 + 31) s
 // 3: bf16, used as it is (a16w16, bf16 K).  4: bf16, quantized here per
 // head row (the per-tensor rule with the row as the tensor; fp8 or fp4 K), so
 // no tensor-wide amax pass has to run first.  5: as 4, the work-group's item
-// planned here by the block (65 to 256 query rows).
+// planned here by the block (65 to 256 query rows).  6: as 1, planned here as 4,
+// with the tensor's |q| maximum taken here from the whole of Q (a few rows, see
+// kSelfAmaxRows): no amax launch.
 template <int KF, int VF, bool IDX, int QM>
 __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_kernel(const DecodeParams p) {
   using C = H16<KF, VF>;
@@ -186,15 +188,15 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
 
   const int32_t* plan = p.plan;
   int4 it;
-  if (QM == 5 || (QM == 4 && p.plan_here)) {  // only the per-row Q route plans here
-    // QM 4, up to 64 rows: wave 0 plans in registers and takes this
+  if (QM == 5 || ((QM == 4 || QM == 6) && p.plan_here)) {
+    // QM 4 and 6, up to 64 rows: wave 0 plans in registers and takes this
     // work-group's item; QM 5, up to 256: the block plans (its scratch on the
     // ring, which nothing has written yet) and the thread of the item's row
     // takes it (a variant of its own, so that the small batches' kernel does
     // not carry the block planner's code).  Work-group 0 also writes what the
     // combine reads of the plan.
     __shared__ int4 s_item;
-    if constexpr (QM == 4) {
+    if constexpr (QM == 4 || QM == 6) {
       if ((threadIdx.x >> 6) == 0) {
         const WavePlan P = plan_wave(p.kv_indptr, p.batch, p.plan_qlen, p.plan_target, p.plan_min_chunk,
                                      p.plan_max_splits);
@@ -229,6 +231,9 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
     __syncthreads();
     it = s_item;
     if (it.x < 0) return;  // past the plan's items (block-uniform)
+    if constexpr (QM == 6) {  // the plan a call leaves in the workspace is whole
+      if (threadIdx.x == 0) reinterpret_cast<int4*>(const_cast<int32_t*>(plan) + kPlanHeader)[blockIdx.x] = it;
+    }
   } else {
     if ((int)blockIdx.x >= plan[0]) return;
     it = reinterpret_cast<const int4*>(plan + kPlanHeader)[blockIdx.x];
@@ -440,6 +445,22 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
     for (int k = w; k < QNV / 64; k += 4) dma16_to_lds(src + 1024 * k + 16 * lane, qlds + 1024 * k);
     if constexpr (QM == 1)
       for (int i = tid; i < p.q_nparts; i += 256) qm = max(qm, p.q_partials[i]);
+    if constexpr (QM == 6) {
+      // the whole of Q, four rows (18 vectors a thread) in flight at a time
+      const uint4* qall = reinterpret_cast<const uint4*>(p.q_bf16);
+      const int nv = p.batch * (16 * kQKDim / 8);
+      for (int i0 = 0; i0 < nv; i0 += 18 * 256) {
+        uint4 v[18];
+#pragma unroll
+        for (int k = 0; k < 18; ++k) v[k] = qall[min(i0 + 256 * k + tid, nv - 1)];
+#pragma unroll
+        for (int k = 0; k < 18; ++k) {
+          const uint32_t wv[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) qm = max(qm, max(wv[e] & 0x7FFFu, (wv[e] >> 16) & 0x7FFFu));
+        }
+      }
+    }
     (void)qm;
   } else {
     load_q(p.q_fp8 + ((int64_t)b * 16 + l16) * kQKDim);
@@ -1067,9 +1088,17 @@ static hipError_t launch_decode_t(const DecodeParams& p, int kv_mode, int grid, 
       }
       return hipGetLastError();
     }
-    if (QB && p.q_nparts == 0) {  // bf16 Q with no tensor-wide scale: a16w8, fp8 K only
+    if (QB && p.q_nparts == 0 && !p.plan_here) {  // bf16 Q with no tensor-wide scale: a16w8, fp8 K only
       if (kv_mode != 0) return hipErrorInvalidValue;
       hipLaunchKernelGGL((decode_h16_kernel<0, 0, IDX, 2>), dim3(grid), dim3(256), 0, stream, p);
+      return hipGetLastError();
+    }
+    if (QB && p.plan_here) {  // a few rows: planned and scaled in the kernel
+      switch (kv_mode) {
+        case 0: hipLaunchKernelGGL((decode_h16_kernel<0, 0, IDX, 6>), dim3(grid), dim3(256), 0, stream, p); break;
+        case 1: hipLaunchKernelGGL((decode_h16_kernel<1, 2, IDX, 6>), dim3(grid), dim3(256), 0, stream, p); break;
+        default: return hipErrorInvalidValue;
+      }
       return hipGetLastError();
     }
     constexpr int QM = QB ? 1 : 0;

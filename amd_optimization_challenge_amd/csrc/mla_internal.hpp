@@ -45,6 +45,14 @@ struct PlanTarget {
 // partial write, combine input) exceed their work
 constexpr int kPlanMinChunk = 128;
 
+// Most query rows of which every 16-head work-group takes the per-tensor |q|
+// maximum itself instead of waiting for the amax + plan launch: the rows are 18
+// KiB each for every work-group, from L2, beside the loads of its prologue.  Whole
+// calls, with the launch / without: 4 x 256 tokens 15.5 / 13.0 us, 8 x 8192
+// scattered 33.0 / 28.3; past the line it turns, as every work-group of a long
+// batch reads them all: 16 x 8192 27.9 / 28.6, 32 x 8192 scattered 41.1 / 49.8.
+constexpr int kSelfAmaxRows = 8;
+
 int target_items_for(int batch, int num_heads, int kv_mode, int num_cu);
 PlanTarget plan_target_for(int batch, int num_heads, int kv_mode, int num_cu, bool contiguous);
 WsLayout workspace_layout(int batch, int num_heads, int kv_mode, int num_cu);
