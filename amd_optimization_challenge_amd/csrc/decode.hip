@@ -137,14 +137,17 @@ struct H16 {
   // (two caches) runs one work-group per CU.
   static constexpr int S = KF != 1 ? 2 : (VF == 1 ? 2 : 3);
   static constexpr int BLOCKS_PER_CU = (VF == 1 || KF == 2) ? 1 : 2;
-  // DMA issue: waves RW0..3 gather rows.  fp4 K + fp8 V: wave 0 gathers the
-  // scales of every token.  fp4 K = V: every wave gathers rows and one scale
-  // dword column, wave 3, which has a row window less, a second one, so every
-  // wave issues the same number
-  static constexpr int RW0 = (KF == 1 && VF == 1) ? 1 : 0;
-  static constexpr int NRW = 4 - RW0;
-  static constexpr int NA = (NW + NRW - 1) / NRW;              // windows per row wave: NA or NA - 1
-  static constexpr int NAW = NW % NRW == 0 ? NRW : NW % NRW;   // row waves (from RW0) that issue NA
+  // DMA issue: wave w gathers the row windows w, w + 4, .. of K and of V (two
+  // caches), and of the scales dword column w, wave 3 (a K window short) also the
+  // fifth: every wave but wave 0 issues the same number.  (Two caches: three waves
+  // with all the rows and one with all the scales took 60.8 us where this takes
+  // 55.9 at 64 x 4096 scattered, 56.9 / 48.8 contiguous.)
+  static constexpr int NK = (KW + 3) / 4, NKW = KW % 4;  // K windows per wave; waves that issue NK (else NK - 1)
+  static constexpr int NV = (VW + 3) / 4, NVW = VW % 4;  // of V (VF == 1)
+  static constexpr int per_group(int w) {                // DMAs of a group, less wave 0's slots
+    return NK - (w >= NKW) + (VW > 0 ? NV - (w >= NVW) : 0) + (KF == 1 ? 1 + (w == 3) : 0);
+  }
+  static_assert(per_group(1) == per_group(2) && per_group(2) == per_group(3), "waves 1 to 3 alike");
   static constexpr bool VB16 = VF == 2;                        // fp4 V, bf16 PV from registers
   static constexpr bool PB = VF >= 2;                          // P shared as bf16 [head][token] (bf16 PV)
   static constexpr int PST = 144;                              // its row stride in bytes: 64 tokens + 16
@@ -275,76 +278,72 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
   // every address)
   constexpr int64_t kFarStride = 1 << 24;
   constexpr bool kNear = !IDX && QM != 2;
-  const bool near_rows = kNear && p.k_row_stride <= kFarStride && (KF != 1 || p.k_scale_stride <= kFarStride);
-  uint32_t voff[C::VW == 0 && (kNear || QM == 2) ? C::NA : 1];
-  if constexpr (C::VW == 0 && (kNear || QM == 2)) {
+  const bool near_rows = kNear && p.k_row_stride <= kFarStride && (KF != 1 || p.k_scale_stride <= kFarStride) &&
+                         (VF != 1 || p.v_row_stride <= kFarStride);
+  // source of K (V) window k's chunk inside the tile: its row's offset if near,
+  // and the 16-byte chunk of the row (the last one pads)
+  uint32_t voff[kNear || QM == 2 ? C::NK : 1], vvoff[kNear && C::VW > 0 ? C::NV : 1];
+  if constexpr (kNear || QM == 2) {
 #pragma unroll
-    for (int k = 0; k < C::NA; ++k) {
+    for (int k = 0; k < C::NK; ++k) {
       const int e = 64 * (w + 4 * k) + lane, tok = e / C::KCPR, ch = e - tok * C::KCPR;
       voff[k] = (kNear ? (uint32_t)tok * (uint32_t)p.k_row_stride : 0u) + (uint32_t)(16 * min(ch, C::KCH - 1));
     }
   }
+  if constexpr (kNear && C::VW > 0) {
+#pragma unroll
+    for (int k = 0; k < C::NV; ++k) {
+      const int e = 64 * (w + 4 * k) + lane, tok = e / C::VCPR, ch = e - tok * C::VCPR;
+      vvoff[k] = (uint32_t)tok * (uint32_t)p.v_row_stride + (uint32_t)(16 * min(ch, 31));
+    }
+  }
   auto issue_rows = [&](int t, int st, int ss) __attribute__((always_inline)) {
-    if constexpr (C::VW == 0) {
-      // windows u = w + 4k of the stage; the last one (k = NA - 1) on waves below NAW
-      static_assert(C::RW0 == 0, "every wave gathers rows");
-      const uint32_t base = __builtin_amdgcn_readfirstlane(lds0 + st * C::STAGE + 1024 * w);
-      if constexpr (kNear) {
-        if (near_rows && kTile * (t + 1) <= ntok) {
-          const uint8_t* sb = p.k_cache + (int64_t)(t_beg + kTile * t) * p.k_row_stride;
-          dma16_windows<0, C::NA - 1>(base, [&](auto k) __attribute__((always_inline)) { return voff[decltype(k)::value]; }, sb);
-          if (w < C::NAW) dma16_windows<C::NA - 1, C::NA>(base, [&](auto k) __attribute__((always_inline)) { return voff[decltype(k)::value]; }, sb);
-          return;
+    const uint32_t base = __builtin_amdgcn_readfirstlane(lds0 + st * C::STAGE + 1024 * w);
+    const uint32_t vbase = base + 1024 * C::KW;
+    if constexpr (kNear) {
+      if (near_rows && kTile * (t + 1) <= ntok) {
+        auto off = [&](auto k) __attribute__((always_inline)) { return voff[decltype(k)::value]; };
+        const uint8_t* sb = p.k_cache + (int64_t)(t_beg + kTile * t) * p.k_row_stride;
+        dma16_windows<0, C::NK - 1>(base, off, sb);
+        if (w < C::NKW) dma16_windows<C::NK - 1, C::NK>(base, off, sb);
+        if constexpr (C::VW > 0) {
+          auto offv = [&](auto k) __attribute__((always_inline)) { return vvoff[decltype(k)::value]; };
+          const uint8_t* sv = p.v_cache + (int64_t)(t_beg + kTile * t) * p.v_row_stride;
+          dma16_windows<0, C::NV - 1>(vbase, offv, sv);
+          if (w < C::NVW) dma16_windows<C::NV - 1, C::NV>(vbase, offv, sv);
         }
+        return;
       }
-      // all slot reads first (each DMA block below is an asm barrier for memory
-      // ops), the addresses as each block needs them
-      int sl[C::NA];
+    }
+    // all slot reads first (each DMA block below is an asm barrier for memory
+    // ops), the addresses as each block needs them
+    int sl[C::NK], slv[C::VW > 0 ? C::NV : 1];
 #pragma unroll
-      for (int k = 0; k < C::NA; ++k) sl[k] = slot_of(t, ss, min(64 * (w + 4 * k) + lane, kTile * C::KCPR - 1) / C::KCPR);
-      auto row_addr = [&](auto kt) __attribute__((always_inline)) {
+    for (int k = 0; k < C::NK; ++k) sl[k] = slot_of(t, ss, min(64 * (w + 4 * k) + lane, kTile * C::KCPR - 1) / C::KCPR);
+    if constexpr (C::VW > 0) {
+#pragma unroll
+      for (int k = 0; k < C::NV; ++k) slv[k] = slot_of(t, ss, min(64 * (w + 4 * k) + lane, kTile * C::VCPR - 1) / C::VCPR);
+    }
+    auto row_addr = [&](auto kt) __attribute__((always_inline)) {
+      constexpr int k = decltype(kt)::value;
+      uint32_t co = (uint32_t)(16 * min((64 * (w + 4 * k) + lane) % C::KCPR, C::KCH - 1));
+      if constexpr (QM == 2) {  // a 32-bit offset kept per window, not the 64-bit base + offset
+        asm volatile("" : "+v"(voff[k]));
+        co = voff[k];
+      }
+      // slot x stride in one v_mad_u64_u32 (both below 2^31, checked on the host)
+      return p.k_cache + ((uint64_t)(uint32_t)sl[k] * (uint32_t)p.k_row_stride + co);
+    };
+    dma16_windows<0, C::NK - 1>(base, row_addr);
+    if (w < C::NKW) dma16_windows<C::NK - 1, C::NK>(base, row_addr);
+    if constexpr (C::VW > 0) {
+      auto v_addr = [&](auto kt) __attribute__((always_inline)) {
         constexpr int k = decltype(kt)::value;
-        // 16-B chunk of the row (the last one pads)
-        uint32_t co = (uint32_t)(16 * min((64 * (w + 4 * k) + lane) % C::KCPR, C::KCH - 1));
-        if constexpr (QM == 2) {  // a 32-bit offset kept per window, not the 64-bit base + offset
-          asm volatile("" : "+v"(voff[k]));
-          co = voff[k];
-        }
-        // slot x stride in one v_mad_u64_u32 (both below 2^31, checked on the host)
-        return p.k_cache + ((uint64_t)(uint32_t)sl[k] * (uint32_t)p.k_row_stride + co);
+        return p.v_cache + ((uint64_t)(uint32_t)slv[k] * (uint32_t)p.v_row_stride +
+                            (uint32_t)(16 * min((64 * (w + 4 * k) + lane) % C::VCPR, 31)));
       };
-      dma16_windows<0, C::NA - 1>(base, row_addr);
-      if (w < C::NAW) dma16_windows<C::NA - 1, C::NA>(base, row_addr);
-    } else {  // two caches: row waves, windows u = (w - RW0) + NRW k, K rows then V rows
-      if (w < C::RW0) return;
-      const uint32_t sbase = lds0 + st * C::STAGE;
-      // all slot reads first: each DMA below is an asm barrier for memory ops
-      int sl[C::NA], co[C::NA];
-#pragma unroll
-      for (int k = 0; k < C::NA; ++k) {
-        const int u = (w - C::RW0) + C::NRW * k;
-        if (u < C::KW) {
-          const int e = 64 * u + lane;  // 16-B chunk index within the stage
-          const int tok = e / C::KCPR, ch = e - tok * C::KCPR;
-          sl[k] = slot_of(t, ss, tok);
-          co[k] = 16 * min(ch, C::KCH - 1);
-        } else if (u < C::NW) {
-          const int e = 64 * (u - C::KW) + lane;
-          const int tok = e / C::VCPR, ch = e - tok * C::VCPR;
-          sl[k] = slot_of(t, ss, tok);
-          co[k] = 16 * min(ch, 31);
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < C::NA; ++k) {
-        const int u = (w - C::RW0) + C::NRW * k;
-        if (u < C::KW)
-          dma16_to_lds_nt(p.k_cache + ((uint64_t)(uint32_t)sl[k] * (uint32_t)p.k_row_stride + (uint32_t)co[k]),
-                       sbase + 1024 * u);
-        else if (u < C::NW)
-          dma16_to_lds_nt(p.v_cache + ((uint64_t)(uint32_t)sl[k] * (uint32_t)p.v_row_stride + (uint32_t)co[k]),
-                       sbase + 1024 * u);
-      }
+      dma16_windows<0, C::NV - 1>(vbase, v_addr);
+      if (w < C::NVW) dma16_windows<C::NV - 1, C::NV>(vbase, v_addr);
     }
   };
   // fp4 K scales: the 18 e8m0 bytes of token `lane` of tile t as 5 dwords
@@ -356,39 +355,19 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
   auto issue_scales = [&](int t, int st, int ss) __attribute__((always_inline)) {
     if constexpr (KF == 1) {
       const uint32_t sb = lds0 + C::OFF_SC + st * C::SCST;
-      if constexpr (C::VW == 0) {  // column w, and the last one on wave 3
-        const uint8_t* srow;
-        if (near_rows && kTile * (t + 1) <= ntok)
-          srow = p.k_scales + (int64_t)(t_beg + kTile * t) * p.k_scale_stride + (uint32_t)lane * (uint32_t)p.k_scale_stride;
-        else
-          srow = p.k_scales + (uint64_t)(uint32_t)slot_of(t, ss, lane) * (uint32_t)p.k_scale_stride;
-        dma4_to_lds(srow + 4 * w, sb + 256 * w);
-        if (w == 3) dma4_to_lds(srow + 14, sb + 256 * 4);
-      } else if (w == 0) {
-        const uint8_t* srow = p.k_scales + (uint64_t)(uint32_t)slot_of(t, ss, lane) * (uint32_t)p.k_scale_stride;
-#pragma unroll
-        for (int j = 0; j < kScWin; ++j) dma4_to_lds(srow + (j < 4 ? 4 * j : 14), sb + 256 * j);
-      }
+      const uint8_t* srow;  // column w, and the fifth on wave 3
+      if (near_rows && kTile * (t + 1) <= ntok)
+        srow = p.k_scales + (int64_t)(t_beg + kTile * t) * p.k_scale_stride + (uint32_t)lane * (uint32_t)p.k_scale_stride;
+      else
+        srow = p.k_scales + (uint64_t)(uint32_t)slot_of(t, ss, lane) * (uint32_t)p.k_scale_stride;
+      dma4_to_lds(srow + 4 * w, sb + 256 * w);
+      if (w == 3) dma4_to_lds(srow + 14, sb + 256 * 4);
     }
   };
   // this wave's wait for tile t's rows (and scales), k groups issued after them
   auto wait_tile = [&](int k) __attribute__((always_inline)) {
-    constexpr int SL = IDX ? 1 : 0;  // wave 0 issues one slot DMA per group
-    if constexpr (KF == 1 && C::VW == 0) {
-      // NA rows and one scale column, or NA - 1 rows and two (wave 3)
-      static_assert(C::NAW == 3 && kScWin == 5, "per-wave DMA counts");
-      if (IDX && w == 0) wait_groups<C::NA + 1 + SL>(k);
-      else wait_groups<C::NA + 1>(k);
-    } else if constexpr (KF == 1) {
-      // wave 0: one slot DMA + the 5 scale DMAs per group
-      if (w == 0) wait_groups<kScWin + SL>(k);
-      else if (w - C::RW0 < C::NAW) wait_groups<C::NA>(k);
-      else wait_groups<C::NA - 1>(k);
-    } else {
-      static_assert(C::NAW == 1, "only wave 0 has the last window");
-      if (w == 0) wait_groups<C::NA + SL>(k);
-      else wait_groups<C::NA - 1>(k);
-    }
+    if (w == 0) wait_groups<C::per_group(0) + (IDX ? 1 : 0)>(k);  // and a slot DMA per group
+    else wait_groups<C::per_group(1)>(k);
   };
   // group x = {slots(x + S), rows(x) | scales(x)}.  The prologue issues groups
   // 0 .. S-1 (every stage is free then, so the first S tiles are in flight

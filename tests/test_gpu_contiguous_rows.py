@@ -24,7 +24,7 @@ def _far(t, rows):
     return out
 
 
-@pytest.mark.parametrize("mode", ["fp8", "mxfp4", "bf16"])
+@pytest.mark.parametrize("mode", ["fp8", "mxfp4", "mxfp4k_fp8v", "bf16"])
 @pytest.mark.parametrize("lens", [[1], [64], [63, 2], [65, 1], [128], [1, 64, 127]])
 def test_near_and_far_rows(mode, lens):
     case = M.host_case(lens, 16, mode, seed=sum(lens), permute=False)
@@ -33,11 +33,11 @@ def test_near_and_far_rows(mode, lens):
     data = M.device_data(q, kv, indptr, idx, caches, mode, sm, pass_indices=False)
     near = custom_kernel(data).clone()
     kvd, T = data[1], kv.shape[0]
-    if mode == "fp8":
+    if "fp8" in kvd:
         kvd["fp8"] = (_far(kvd["fp8"][0], T), kvd["fp8"][1])
-    elif mode == "mxfp4":
+    if "mxfp4" in kvd:
         kvd["mxfp4"] = (_far(kvd["mxfp4"][0], T), kvd["mxfp4"][1])
-    else:
+    if mode == "bf16":
         kvd["bf16"] = _far(kvd["bf16"], T).view(torch.bfloat16)
     far = custom_kernel(data)
     assert torch.equal(near.view(torch.int16), far.view(torch.int16))
