@@ -178,6 +178,17 @@ static bool rows_as_one_item(int q_seq_len, int num_heads, int kv_mode) {
   return num_heads == 16 && kv_mode == MLA_KV_FP8 && q_seq_len >= 2 && q_seq_len <= kMaxRowsPerItem;
 }
 
+// The decode plans its own work in the kernel; returns its grid (the planner
+// keeps within the target plus the rows).
+static int plan_in_kernel(DecodeParams* p, const WsLayout& L, const PlanTarget& t, int qlen) {
+  p->plan_here = 1;
+  p->plan_qlen = qlen;
+  p->plan_target = t.items;
+  p->plan_min_chunk = t.min_chunk;
+  p->plan_max_splits = t.max_splits;
+  return t.items + p->batch < L.max_items ? t.items + p->batch : L.max_items;
+}
+
 namespace {
 
 int decode_params(const void* q_fp8, const float* q_scale, const void* k_cache, int64_t k_row_stride,
@@ -241,6 +252,7 @@ int decode_params(const void* q_fp8, const float* q_scale, const void* k_cache, 
   p->q_partials = nullptr;
   p->q_nparts = 0;
   p->q_per_row = 0;
+  p->q_self_amax = 0;
   p->plan_here = 0;
   p->plan_qlen = 1;
   p->plan_target = 0;
@@ -481,12 +493,14 @@ int mla_decode_fwd(const void* q_bf16, const void* k_cache, int64_t k_row_stride
   uint32_t* partials = reinterpret_cast<uint32_t*>(ws + L.quant_off);
   int nb = 0;
   if (kv_mode == MLA_KV_BF16) {  // a16w16: Q is used as it is, no amax pass
-    hipError_t e = launch_plan(kv_indptr, batch, q_seq_len,
-                               plan_target_for(batch, num_heads, kv_mode, ncu, kv_indices == nullptr),
-                               L.max_items, reinterpret_cast<int32_t*>(ws + L.plan_off), s);
+    const PlanTarget t = plan_target_for(batch, num_heads, kv_mode, ncu, kv_indices == nullptr);
+    int grid = L.max_items;
+    hipError_t e = hipSuccess;
+    if (batch <= kWavePlanRows) grid = plan_in_kernel(&p, L, t, q_seq_len);
+    else e = launch_plan(kv_indptr, batch, q_seq_len, t, L.max_items, reinterpret_cast<int32_t*>(ws + L.plan_off), s);
     if (e != hipSuccess) return hip_fail(e, "plan launch");
     p.q_bf16 = static_cast<const uint16_t*>(q_bf16);
-    e = launch_decode(p, kv_mode, L.max_items, s);
+    e = launch_decode(p, kv_mode, grid, s);
     if (e != hipSuccess) return hip_fail(e, "decode launch");
     e = launch_combine(p, s);
     if (e != hipSuccess) return hip_fail(e, "combine launch");
@@ -496,12 +510,8 @@ int mla_decode_fwd(const void* q_bf16, const void* k_cache, int64_t k_row_stride
     // the decode plans its own work and scales its own Q: one launch fewer
     const PlanTarget t = plan_target_for(batch, num_heads, kv_mode, ncu, kv_indices == nullptr);
     p.q_bf16 = static_cast<const uint16_t*>(q_bf16);
-    p.plan_here = 1;
-    p.plan_qlen = q_seq_len;
-    p.plan_target = t.items;
-    p.plan_min_chunk = t.min_chunk;
-    p.plan_max_splits = t.max_splits;
-    hipError_t e = launch_decode(p, kv_mode, t.items + batch < L.max_items ? t.items + batch : L.max_items, s);
+    p.q_self_amax = 1;
+    hipError_t e = launch_decode(p, kv_mode, plan_in_kernel(&p, L, t, q_seq_len), s);
     if (e != hipSuccess) return hip_fail(e, "decode launch");
     e = launch_combine(p, s);
     if (e != hipSuccess) return hip_fail(e, "combine launch");
@@ -603,12 +613,14 @@ int mla_decode_fwd_a16w8(const void* q_bf16, const void* k_cache, int64_t k_row_
                      lse_out, &p, &L);
   if (rc) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  hipError_t e = launch_plan(kv_indptr, batch, q_seq_len,
-                             plan_target_for(batch, num_heads, kv_mode, ncu, kv_indices == nullptr),
-                             L.max_items, reinterpret_cast<int32_t*>(ws + L.plan_off), s);
+  const PlanTarget t = plan_target_for(batch, num_heads, kv_mode, ncu, kv_indices == nullptr);
+  int grid = L.max_items;
+  hipError_t e = hipSuccess;
+  if (batch <= kWavePlanRows) grid = plan_in_kernel(&p, L, t, q_seq_len);
+  else e = launch_plan(kv_indptr, batch, q_seq_len, t, L.max_items, reinterpret_cast<int32_t*>(ws + L.plan_off), s);
   if (e != hipSuccess) return hip_fail(e, "plan launch");
   p.q_bf16 = static_cast<const uint16_t*>(q_bf16);  // no partials: each work-group scales its own Q rows
-  e = launch_decode(p, kv_mode, L.max_items, s);
+  e = launch_decode(p, kv_mode, grid, s);
   if (e != hipSuccess) return hip_fail(e, "decode launch");
   e = launch_combine(p, s);
   if (e != hipSuccess) return hip_fail(e, "combine launch");
@@ -654,12 +666,7 @@ int mla_decode_fwd_rowq(const void* q_bf16, const void* k_cache, int64_t k_row_s
     // the decode plans its own work (one wave up to 64 rows, the block up to
     // 256): one launch fewer; at most max(t.items, batch) items (the chunk
     // search keeps the count within the target, or one piece per row)
-    p.plan_here = 1;
-    p.plan_qlen = q_seq_len;
-    p.plan_target = t.items;
-    p.plan_min_chunk = t.min_chunk;
-    p.plan_max_splits = t.max_splits;
-    grid = t.items + batch < L.max_items ? t.items + batch : L.max_items;
+    grid = plan_in_kernel(&p, L, t, q_seq_len);
   } else {
     e = launch_plan(kv_indptr, batch, q_seq_len, t, L.max_items, reinterpret_cast<int32_t*>(ws + L.plan_off), s);
     if (e != hipSuccess) return hip_fail(e, "plan launch");

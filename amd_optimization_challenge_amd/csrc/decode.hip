@@ -179,7 +179,8 @@ constexpr int kVScaleSpan = 31;  // fp4 V: P' = P 2^(e - E_ref) <= 2^(96 + 31) s
 // no tensor-wide amax pass has to run first.  5: as 4, the work-group's item
 // planned here by the block (65 to 256 query rows).  6: as 1, planned here as 4,
 // with the tensor's |q| maximum taken here from the whole of Q (a few rows, see
-// kSelfAmaxRows): no amax launch.
+// kSelfAmaxRows): no amax launch.  2, 3, 4 and 6 plan here in one wave where
+// p.plan_here says so (up to 64 query rows).
 template <int KF, int VF, bool IDX, int QM>
 __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_kernel(const DecodeParams p) {
   using C = H16<KF, VF>;
@@ -191,15 +192,16 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
 
   const int32_t* plan = p.plan;
   int4 it;
-  if (QM == 5 || ((QM == 4 || QM == 6) && p.plan_here)) {
-    // QM 4 and 6, up to 64 rows: wave 0 plans in registers and takes this
+  constexpr bool kWavePlan = QM == 2 || QM == 3 || QM == 4 || QM == 6;
+  if (QM == 5 || (kWavePlan && p.plan_here)) {
+    // up to 64 rows: wave 0 plans in registers and takes this
     // work-group's item; QM 5, up to 256: the block plans (its scratch on the
     // ring, which nothing has written yet) and the thread of the item's row
     // takes it (a variant of its own, so that the small batches' kernel does
     // not carry the block planner's code).  Work-group 0 also writes what the
     // combine reads of the plan.
     __shared__ int4 s_item;
-    if constexpr (QM == 4 || QM == 6) {
+    if constexpr (kWavePlan) {
       if ((threadIdx.x >> 6) == 0) {
         const WavePlan P = plan_wave(p.kv_indptr, p.batch, p.plan_qlen, p.plan_target, p.plan_min_chunk,
                                      p.plan_max_splits);
@@ -234,7 +236,7 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
     __syncthreads();
     it = s_item;
     if (it.x < 0) return;  // past the plan's items (block-uniform)
-    if constexpr (QM == 6) {  // the plan a call leaves in the workspace is whole
+    if constexpr (kWavePlan && QM != 4) {  // the plan a call leaves in the workspace is whole
       if (threadIdx.x == 0) reinterpret_cast<int4*>(const_cast<int32_t*>(plan) + kPlanHeader)[blockIdx.x] = it;
     }
   } else {
@@ -1079,12 +1081,12 @@ static hipError_t launch_decode_t(const DecodeParams& p, int kv_mode, int grid, 
       }
       return hipGetLastError();
     }
-    if (QB && p.q_nparts == 0 && !p.plan_here) {  // bf16 Q with no tensor-wide scale: a16w8, fp8 K only
+    if (QB && p.q_nparts == 0 && !p.q_self_amax) {  // bf16 Q with no tensor-wide scale: a16w8, fp8 K only
       if (kv_mode != 0) return hipErrorInvalidValue;
       hipLaunchKernelGGL((decode_h16_kernel<0, 0, IDX, 2>), dim3(grid), dim3(256), 0, stream, p);
       return hipGetLastError();
     }
-    if (QB && p.plan_here) {  // a few rows: planned and scaled in the kernel
+    if (QB && p.plan_here && p.q_self_amax) {  // a few rows: planned and scaled in the kernel
       switch (kv_mode) {
         case 0: hipLaunchKernelGGL((decode_h16_kernel<0, 0, IDX, 6>), dim3(grid), dim3(256), 0, stream, p); break;
         case 1: hipLaunchKernelGGL((decode_h16_kernel<1, 2, IDX, 6>), dim3(grid), dim3(256), 0, stream, p); break;

@@ -56,6 +56,7 @@ struct DecodeParams {
   // and split cap, and its work-group 0 writes the rows' piece counts and the
   // header the combine reads (plan then points at writable workspace)
   int q_per_row;
+  int q_self_amax;  // per-tensor scale from the maximum the kernel takes itself (needs plan_here)
   int plan_here;
   int plan_qlen;
   int plan_target;

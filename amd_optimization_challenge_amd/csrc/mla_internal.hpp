@@ -45,6 +45,10 @@ struct PlanTarget {
 // partial write, combine input) exceed their work
 constexpr int kPlanMinChunk = 128;
 
+// Most query rows that one wave plans (mla_plan.hpp): up to there the bf16-Q routes
+// plan in the decode instead of in a launch of their own before it, whose 3 to 5
+// us are gone for about 1 us at the decode's start.
+constexpr int kWavePlanRows = 64;
 // Most query rows of which every 16-head work-group takes the per-tensor |q|
 // maximum itself instead of waiting for the amax + plan launch: the rows are 18
 // KiB each for every work-group, from L2, beside the loads of its prologue.  Whole
