@@ -967,7 +967,7 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
 // the split partials are read in batches of 8 so their loads overlap.  PG
 // groups of 256 threads take the batches in turn and merge through LDS at the
 // end: a chain of dependent batches is all a small grid does (4 rows of 32
-// pieces are 16 blocks), so where the grid leaves CUs without a block PG = 4
+// pieces are 16 blocks), so where the grid leaves most CUs without a block PG = 4
 // runs four batches side by side (32 pieces of 4 rows: 5.9 -> 4.6 us; at most 8
 // pieces, where the other groups leave at once, as before: 2.4 to 3.8).
 // ============================================================================
@@ -1124,8 +1124,10 @@ hipError_t launch_decode(const DecodeParams& p, int kv_mode, int grid, hipStream
 
 hipError_t launch_combine(const DecodeParams& p, hipStream_t stream) {
   const dim3 grid(p.batch, p.num_heads / 16, 4);
-  // fewer blocks than CUs (gfx950: 256)
-  if (p.batch <= 64 && p.batch * (p.num_heads / 16) * 4 <= 256)
+  // up to a block per four CUs (gfx950: 256): rows few enough to be cut into more
+  // than 8 pieces; with more blocks 1024-thread ones start later than they save
+  // (32 x 1024, 8 pieces: 3.4 us in small blocks, 3.8 in large ones)
+  if (p.batch <= 16 && p.batch * (p.num_heads / 16) * 4 <= 64)
     hipLaunchKernelGGL((combine_kernel<4>), grid, dim3(1024), 0, stream, p);
   else
     hipLaunchKernelGGL((combine_kernel<1>), grid, dim3(256), 0, stream, p);
