@@ -28,18 +28,17 @@
 // to six slots ahead of their MFMA, one of 22 softmax steps, one row DMA every
 // two or three slots of the pair.  Addresses move once per tile, in place.
 //
-// LDS: a 4-stage ring of 64-row pairs (608-byte rows: 576 + 32 of padding,
-// 16-byte chunks of row r XOR-swizzled by (r >> 2) & 7, which keeps both the K
-// fragment reads (ds_read_b128) and the V^T transpose reads
-// (ds_read_b64_tr_b8) near their bank-conflict floor).  Rows arrive by LDS-DMA
+// LDS: a 4-stage ring of 64-row pairs in the row layout of mla_tile64.hpp (576-byte
+// rows, chunks swizzled; padded 608-byte rows cost two more DMA windows
+// a pair and ten more address registers to move: 64 x 4000 keys 60.1 us of decode
+// with them, 56.9 without; 256 x 1024 58.3 and 56.6).  Rows arrive by LDS-DMA
 // (global_load_lds_dwordx4) two pairs ahead of use; a pair's 64 slot indices
 // arrive by one dword LDS-DMA four pairs ahead of its rows.  Two work-group
 // barriers per pair: one once every wave has read the last V^T of pair q - 2
 // (its stage then takes pair q + 2's rows), one once pair q + 1 has landed.
 // The LDS-DMA writes lane l of a 1 KiB window to position 64u + l of the
-// pair's stage, so each lane fetches whichever chunk its position holds
-// (padding positions re-fetch chunk 0 of their row, a cache hit).  Q comes the
-// same way, into stages 2-3 before the first rows(2) land there.
+// pair's stage, so each lane fetches whichever chunk its position holds.  Q comes
+// the same way, into stages 2-3 before the first rows(2) land there.
 //
 // Softmax: per head a reference m_ref (the first tile's ceil max); a tile's
 // P' = 2^(c s - m_t + 8) with m_t its ceil max, and the PV MFMA's e8m0 B scale
@@ -83,19 +82,19 @@ constexpr float kRebaseF = 96.0f;
 
 struct G128 {
   static constexpr int RST = kRowSt;            // LDS row stride
-  static constexpr int CPR = RST / 16;          // 38 chunk positions per row (36 used)
+  static constexpr int CPR = kRowCh;            // 36 chunks
   static constexpr int HT = 32;                 // tokens per tile
-  static constexpr int TSTAGE = HT * RST;       // 19456 B per tile
-  static constexpr int PSTAGE = 2 * TSTAGE;     // a pair of tiles: 38 one-KiB DMA windows
+  static constexpr int TSTAGE = HT * RST;       // 18432 B per tile
+  static constexpr int PSTAGE = 2 * TSTAGE;     // a pair of tiles: 36 one-KiB DMA windows
   static constexpr int WIN = PSTAGE / 1024;
   static constexpr int NP = 4;                  // pair stages: pairs q-1 (V), q (K), q+1, q+2 (in flight)
   static constexpr int NSL = 8;                 // slot stages (one per pair)
-  static constexpr int DMAX = (WIN + 3) / 4;    // windows of waves 0, 1 (waves 2, 3: DMAX - 1)
+  static constexpr int DMAX = WIN / 4;          // windows per wave
   static constexpr int OFF_SLOT = NP * PSTAGE;
   static constexpr int OFF_FLAG = OFF_SLOT + NSL * 256;  // [4] per-wave overflow flags
   static constexpr int LDS = OFF_FLAG + 16;
   static constexpr int OFF_Q = 2 * PSTAGE;      // Q (prologue): pair stages 2-3
-  static_assert(WIN == 38 && DMAX == 10, "DMA window split");
+  static_assert(4 * DMAX == WIN && 128 * kQKDim <= 2 * PSTAGE, "DMA window split, Q staging");
   static_assert(LDS <= 160 * 1024, "LDS");
 };
 
@@ -246,12 +245,12 @@ struct H128Sched {
   static constexpr int kStageFree = 20;
   static constexpr int dma_slot(int k) { return 21 + 5 * (k / 2) + 2 * (k % 2); }
   static constexpr int row_dma(int s) {
-    for (int k = 0; k < 10; ++k)
+    for (int k = 0; k < G128::DMAX; ++k)
       if (dma_slot(k) == s) return k;
     return -1;
   }
   static constexpr int row_read(int s) {
-    for (int k = 0; k < 10; ++k)
+    for (int k = 0; k < G128::DMAX; ++k)
       if (dma_slot(k) - 2 == s) return k;
     return -1;
   }
@@ -397,16 +396,15 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
 
   // ---- DMA maps ---------------------------------------------------------------
   // fp8 cache: window u = w + 4k of a pair stage puts lane l at chunk position
-  // 64u + l = (row r of the pair, position j); it fetches logical chunk
-  // g128_pos(r, j) (chunk 0 for the two padding positions); packed (r << 10 |
-  // byte offset), two windows per register.
+  // 64u + l = (row r of the pair, position j); it fetches logical chunk j ^
+  // row_key(r); packed (r << 10 | byte offset), two windows per register.
   // Two-cache mode: window m of each type (the wave's window u = w + 4m of the
   // stage) puts lane l at position e = 64u + l: K, chunk e of the stage = row
   // e / 19, chunk e % 19 (the padding chunk re-fetches chunk 0); V half, row e /
   // 17, chunk e % 17 (likewise); e8m0, plane u, row l: the dword at byte 4u (u <
   // 4) or 14 (u = 4) of the row's scales.  Packed (r << 9 | source byte offset
   // in the row), entries K 0..4, e8m0 5..9, V 10..14.
-  constexpr int kMaps = MIX ? 8 : G128::DMAX / 2;
+  constexpr int kMaps = MIX ? 8 : (G128::DMAX + 1) / 2;
   uint32_t dmap[kMaps];
   if constexpr (MIX) {
     uint32_t ent[16];
@@ -426,9 +424,9 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
   } else {
 #pragma unroll
     for (int k = 0; k < G128::DMAX; ++k) {
-      const int pidx = min(64 * (w + 4 * k) + lane, 64 * G128::WIN - 1);
+      const int pidx = 64 * (w + 4 * k) + lane;
       const int r = pidx / G128::CPR, j = pidx - G128::CPR * r;
-      const uint32_t e = ((uint32_t)r << 10) | (uint32_t)(16 * (j < 36 ? g128_pos(r, j) : 0));
+      const uint32_t e = ((uint32_t)r << 10) | (uint32_t)(16 * (j ^ row_key(r)));
       if (k % 2 == 0) dmap[k / 2] = e;
       else dmap[k / 2] |= e << 16;
     }
@@ -450,17 +448,15 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
     }
   };
   auto row_dma = [&](int k, int sl, uint32_t stage_w) __attribute__((always_inline)) {
-    if (k < G128::DMAX - 1 || w < 2) {
-      asm volatile("" : "+v"(dmap[k / 2]));
-      const uint32_t off = (dmap[k / 2] >> (16 * (k % 2))) & 1023u;
-      const uint8_t* src = p.k_cache + ((uint64_t)(uint32_t)sl * (uint32_t)p.k_row_stride + off);
-      uint32_t saved;  // M0 saved and restored, one wait state before the DMA; nt as in dma16_to_lds_nt
-      asm volatile("s_mov_b32 %0, m0\n\ts_add_u32 m0, %1, %2\n\ts_mov_b32 %0, %0\n\t"
-                   "global_load_lds_dwordx4 %3, off nt\n\ts_mov_b32 m0, %0"
-                   : "=&s"(saved)
-                   : "s"(stage_w), "i"(4096 * k), "v"(src)
-                   : "memory", "scc");
-    }
+    asm volatile("" : "+v"(dmap[k / 2]));
+    const uint32_t off = (dmap[k / 2] >> (16 * (k % 2))) & 1023u;
+    const uint8_t* src = p.k_cache + ((uint64_t)(uint32_t)sl * (uint32_t)p.k_row_stride + off);
+    uint32_t saved;  // M0 saved and restored, one wait state before the DMA; nt as in dma16_to_lds_nt
+    asm volatile("s_mov_b32 %0, m0\n\ts_add_u32 m0, %1, %2\n\ts_mov_b32 %0, %0\n\t"
+                 "global_load_lds_dwordx4 %3, off nt\n\ts_mov_b32 m0, %0"
+                 : "=&s"(saved)
+                 : "s"(stage_w), "i"(4096 * k), "v"(src)
+                 : "memory", "scc");
   };
   auto stage_of = [&](int q) __attribute__((always_inline)) -> uint32_t {  // pair q's stage + 1 KiB w
     return __builtin_amdgcn_readfirstlane(lds0 + (q % G128::NP) * G128::PSTAGE + 1024 * w);
@@ -477,12 +473,10 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
     for (int k = 0; k < G128::DMAX; ++k) row_dma(k, sl[k], stw);
   };
   // rows(q) have landed once the DMAs issued after them are all that is
-  // outstanding: the next pair's slot indices (wave 0) and its rows (ten
-  // windows for waves 0 and 1, nine for waves 2 and 3)
+  // outstanding: the next pair's slot indices (wave 0) and its rows
   auto wait_rows = [&]() __attribute__((always_inline)) {
-    if (w == 0) wait_vmcnt<IDX ? G128::DMAX + 1 : G128::DMAX>();
-    else if (w == 1) wait_vmcnt<G128::DMAX>();
-    else wait_vmcnt<G128::DMAX - 1>();
+    if (IDX && w == 0) wait_vmcnt<G128::DMAX + 1>();
+    else wait_vmcnt<G128::DMAX>();
   };
   // the same near the end of the item, where no rows follow (only the slot
   // indices of wave 0)
@@ -552,13 +546,12 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
 
   // ---- lane-constant fragment offsets -----------------------------------------
   // fp8 cache.  K fragment (QK A operand) of K-step ks: row l32 of the tile,
-  // logical chunks 4ks + 2hh + {0, 1} (ks < 8) or 32 + 2hh + {0, 1} (ks = 8).
-  // Rows r and r + 32 share a key, so the offsets hold for both tiles of a pair.
-  // ka[2 (ks & 1) + j] + 128 (ks >> 1) (ks < 8), ka[4 + j] (ks = 8): LDS
-  // addresses of the current K tile, moved along the ring in place.
+  // logical chunks 4ks + 2hh + {0, 1}.  Rows r and r + 32 share a key, so the
+  // offsets hold for both tiles of a pair.  ka[j] + 64 ks: LDS addresses of the
+  // current K tile, moved along the ring in place.
   // Two-cache mode.  K fragment of step ks: chunk 2ks + hh of row l32 of the
   // tile, at ka[0] + 32ks; the row's e8m0 dword j at ka[1] + 256j.
-  uint32_t ka[MIX ? 2 : 6];
+  uint32_t ka[2];
   // (the init lambdas derive everything from an opaque copy of the lane id, so
   // the addresses are formed where they are needed, not kept live from the entry)
   auto init_ka = [&]() __attribute__((always_inline)) {
@@ -569,13 +562,9 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
       ka[0] = lds0 + r * M128::KST + 16 * h;
       ka[1] = lds0 + M128::OFF_S + 4 * r;
     } else {
-      const int r = ln & 31, h2 = (ln >> 5) * 2, x = g128_key(r);
+      const int r = ln & 31, h2 = (ln >> 5) * 2, x = row_key(r);
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        ka[j] = lds0 + r * G128::RST + 16 * ((h2 + j) ^ x);
-        ka[2 + j] = lds0 + r * G128::RST + 16 * ((4 + h2 + j) ^ x);
-        ka[4 + j] = lds0 + r * G128::RST + 16 * (32 + ((h2 + j) ^ (x & 3)));
-      }
+      for (int j = 0; j < 2; ++j) ka[j] = lds0 + r * G128::RST + 16 * ((h2 + j) ^ x);
     }
   };
   // V^T fragment (PV A operand) of dim tile dt (dims 32dt .. +31) over the 64
@@ -583,13 +572,13 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
   // row T0 + 16cc of the pair's first tile (bytes 8cc .. +7) and of its second
   // tile (bytes 16 + 8cc .. +7), T0 = 8(m >> 2) + 4hh + (m & 3), logical chunk
   // 2dt + (G & 1), byte 8oo: byte 16u + 4q + i <-> token 8q + 4hh + i of tile
-  // u, the order of the lane's own scores.  fp8 cache: row T0 + 16cc has key
-  // x0 ^ 4cc, x0 = T0 >> 2; va[4cc + (dt & 3)] + 128 (dt >> 2) (+ TSTAGE): LDS
-  // addresses of the PV pair's first (second) tile.  Two-cache mode: half rows
+  // u, the order of the lane's own scores.  fp8 cache: the rows T0 + 16cc share
+  // T0's key; va[dt & 1] + 64 (dt >> 1) + 16cc RST (+ TSTAGE): LDS addresses of
+  // the PV pair's first (second) tile.  Two-cache mode: half rows
   // of 17 chunks, unswizzled (the 16 rows T0 fall on 16 distinct chunk
   // positions), so every read of dim tile 8h + g is va[0] + 32g + (32u + 16cc)
   // 272, va[0] in the half stage of the iteration.
-  uint32_t va[MIX ? 1 : 8];
+  uint32_t va[MIX ? 1 : 2];
   auto init_va = [&]() __attribute__((always_inline)) {
     int ln = lane;
     asm volatile("" : "+v"(ln));
@@ -598,13 +587,9 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
     if constexpr (MIX) {  // iteration 0 reads half stage 1 (never by an MFMA)
       va[0] = lds0 + M128::OFF_V + M128::VSTAGE + T0 * M128::VST + 16 * (G & 1) + 8 * oo;
     } else {
-      const int x0 = T0 >> 2;
 #pragma unroll
-      for (int cc = 0; cc < 2; ++cc)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)  // pair -2: stage 2 (never read by an MFMA)
-          va[4 * cc + e] = lds0 + 2 * G128::PSTAGE + (T0 + 16 * cc) * G128::RST +
-                           16 * ((2 * e + (G & 1)) ^ (x0 ^ (4 * cc))) + 8 * oo;
+      for (int e = 0; e < 2; ++e)  // pair -2: stage 2 (never read by an MFMA)
+        va[e] = lds0 + 2 * G128::PSTAGE + T0 * G128::RST + 16 * ((2 * e + (G & 1)) ^ row_key(T0)) + 8 * oo;
     }
   };
   typedef __attribute__((address_space(3))) v4i lds_v4i;
@@ -620,10 +605,8 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
     if constexpr (MIX) {
       kf4[g % 3] = *(const lds_v4i*)(uintptr_t)(ka[0] + 32 * g);
     } else {
-      const uint32_t a0 = g < 8 ? ka[2 * (g & 1)] + 128 * (g >> 1) : ka[4];
-      const uint32_t a1 = g < 8 ? ka[2 * (g & 1) + 1] + 128 * (g >> 1) : ka[5];
-      const v4i lo = *(const lds_v4i*)(uintptr_t)a0;
-      const v4i hi = *(const lds_v4i*)(uintptr_t)a1;
+      const v4i lo = *(const lds_v4i*)(uintptr_t)(ka[0] + 64 * g);
+      const v4i hi = *(const lds_v4i*)(uintptr_t)(ka[1] + 64 * g);
       kf[g % 3] = v8i{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     }
   };
@@ -639,11 +622,11 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
       vf[g % 2] = v8i{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
     } else {
       const int dt = 8 * h + g;
-      const uint32_t a0 = va[dt & 3] + 128 * (dt >> 2), a1 = va[4 + (dt & 3)] + 128 * (dt >> 2);
-      const v2i r0 = lds_read_tr8(a0);
-      const v2i r1 = lds_read_tr8(a1);
-      const v2i r2 = lds_read_tr8(a0 + G128::TSTAGE);
-      const v2i r3 = lds_read_tr8(a1 + G128::TSTAGE);
+      const uint32_t a = va[dt & 1] + 64 * (dt >> 1);
+      const v2i r0 = lds_read_tr8(a);
+      const v2i r1 = lds_read_tr8(a + 16 * G128::RST);
+      const v2i r2 = lds_read_tr8(a + G128::TSTAGE);
+      const v2i r3 = lds_read_tr8(a + G128::TSTAGE + 16 * G128::RST);
       vf[g % 2] = v8i{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
     }
   };
@@ -904,7 +887,7 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
         } else {
           const int dk = IT == 0 ? G128::TSTAGE : (((q + 1) & 3) - (q & 3)) * G128::PSTAGE - G128::TSTAGE;
 #pragma unroll
-          for (int jj = 0; jj < 6; ++jj) {
+          for (int jj = 0; jj < 2; ++jj) {
             ka[jj] += dk;
             asm volatile("" : "+v"(ka[jj]));
           }
@@ -918,7 +901,7 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
       if constexpr (!MIX && IT == 0 && i == SC::kRebaseV) {  // pair q - 2 -> q - 1
         const int dv = (((q - 1) & 3) - ((q - 2) & 3)) * G128::PSTAGE;
 #pragma unroll
-        for (int jj = 0; jj < 8; ++jj) {
+        for (int jj = 0; jj < 2; ++jj) {
           va[jj] += dv;
           asm volatile("" : "+v"(va[jj]));
         }
@@ -983,9 +966,8 @@ __global__ __launch_bounds__(256, 1) void decode_h128_kernel(const DecodeParams 
           wait_vmcnt_w<2 * S0 + 2 * MS::ks_per_pair(0), 2 * MS::ks_per_pair(1), 2 * MS::ks_per_pair(2),
                        2 * MS::ks_per_pair(3)>(w);
         } else {
-          if (w == 0) wait_vmcnt<IDX ? 2 * G128::DMAX + 2 : 2 * G128::DMAX>();
-          else if (w == 1) wait_vmcnt<2 * G128::DMAX>();
-          else wait_vmcnt<2 * G128::DMAX - 2>();
+          if (IDX && w == 0) wait_vmcnt<2 * G128::DMAX + 2>();
+          else wait_vmcnt<2 * G128::DMAX>();
         }
         read_q();
       }

@@ -12,10 +12,7 @@
 // keys: a per-lane limit in the tiles at the sequence's end.
 //
 // One work-group of 8 waves per CU, two to a SIMD.  Tiles of 64 tokens in a 4-stage
-// LDS ring of plain 576-byte rows, their 16-byte chunks XOR-swizzled by (r >> 2) &
-// 3: the 144-dword row stride moves a row 16 banks, so four rows and the four keys
-// cover the banks for the K fragment reads (ds_read_b128) and the V^T transpose
-// reads (ds_read_b64_tr_b8) alike, and no DMA lane is spent on padding.
+// LDS ring, in the row layout of mla_tile64.hpp.
 // Waves 0-3 score tile t while waves 4-7 run the PV of tile t - 1: as four waves
 // doing one after the other, a tile took its whole chain (fragment reads, nine
 // MFMAs, softmax, exchange, sixteen MFMAs), about 2.3 us; side by side 1.2, and
@@ -51,8 +48,7 @@ constexpr float kRebaseR = 96.0f;
 
 struct R64 {
   static constexpr int COLS = 64;
-  static constexpr int RST = kQKDim;                     // LDS row stride
-  static constexpr int CPR = RST / 16;                   // 36 chunks
+  static constexpr int RST = kRowSt, CPR = kRowCh;       // LDS row stride, its chunks
   static constexpr int TSTAGE = 32 * RST;                // 32 rows
   static constexpr int STAGE = 2 * TSTAGE;               // 64 rows
   static constexpr int S = 4, NSL = 4;                   // row stages, slot stages
@@ -68,7 +64,6 @@ struct R64 {
   static_assert(STAGE % 4096 == 0 && COLS * kQKDim <= STAGE, "DMA windows, Q staging");
   static_assert(4 * COLS * OST <= OFF_SLOT && LDS <= 160 * 1024, "LDS");
 };
-__device__ __forceinline__ int r64_key(int r) { return (r >> 2) & 3; }
 
 template <bool IDX>
 __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams p) {
@@ -147,7 +142,7 @@ __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams 
 #pragma unroll
   for (int k = 0; k < C::NA; ++k) {
     const int e = 64 * (w + 4 * k) + lane, r = e / C::CPR, j = e - C::CPR * r;
-    wmap[k] = ((uint32_t)r << 16) | (uint32_t)(16 * (j ^ r64_key(r)));
+    wmap[k] = ((uint32_t)r << 16) | (uint32_t)(16 * (j ^ row_key(r)));
   }
   if (IDX && w8 == 0) wait_vmcnt<QJ>();  // the slots (Q may be in flight)
   lds_barrier();
@@ -182,7 +177,7 @@ __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams 
 #pragma unroll
     for (int j = 0; j < QJ; ++j) {
       const int c16 = (q8 >> 1) + 4 * j;
-      *reinterpret_cast<uint2*>(smem + C::OFF_Q + qc * kQKDim + 16 * (c16 ^ r64_key(qc)) + 8 * (q8 & 1)) =
+      *reinterpret_cast<uint2*>(smem + C::OFF_Q + qc * kQKDim + 16 * (c16 ^ row_key(qc)) + 8 * (q8 & 1)) =
           qc < cols ? quant8_fp8(xq[j], qq) : make_uint2(0, 0);
     }
     c = qs * kvs * p.sm_scale * kLog2eR;
@@ -200,7 +195,7 @@ __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams 
     v8i qv[9];
     {
       const uint8_t* qrow = smem + C::OFF_Q + col * kQKDim;
-      const int x0 = 16 * ((2 * hh) ^ r64_key(col)), x1 = 16 * ((2 * hh + 1) ^ r64_key(col));
+      const int x0 = 16 * ((2 * hh) ^ row_key(col)), x1 = 16 * ((2 * hh + 1) ^ row_key(col));
 #pragma unroll
       for (int ks = 0; ks < 9; ++ks) {
         const uint4 a = *reinterpret_cast<const uint4*>(qrow + x0 + 64 * ks);
@@ -213,7 +208,7 @@ __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams 
     typedef __attribute__((address_space(3))) v4i lds_v4i;
     // K fragment of step ks: chunks 4 ks + 2 hh + {0, 1} of row l32 of the half
     const uint32_t krow = lds0 + th * C::TSTAGE + l32 * C::RST;
-    const uint32_t k0 = krow + 16 * ((2 * hh) ^ r64_key(l32)), k1 = krow + 16 * ((2 * hh + 1) ^ r64_key(l32));
+    const uint32_t k0 = krow + 16 * ((2 * hh) ^ row_key(l32)), k1 = krow + 16 * ((2 * hh + 1) ^ row_key(l32));
     for (;;) {
       for (int t = 0; t <= ntiles; ++t) {
         if (IDX && w8 == 0) {  // the slots of tile t + 2 landed (those of t + 3 may be in flight)
@@ -309,7 +304,7 @@ __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams 
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           const int r = T0 + 16 * cc;
-          va[2 * cc + e] = lds0 + r * C::RST + 16 * (8 * w + ((2 * e + (G & 1)) ^ r64_key(r))) + 8 * oo;
+          va[2 * cc + e] = lds0 + r * C::RST + 16 * (8 * w + ((2 * e + (G & 1)) ^ row_key(r))) + 8 * oo;
         }
     }
     for (;;) {

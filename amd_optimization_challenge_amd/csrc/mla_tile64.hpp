@@ -7,17 +7,15 @@
 
 namespace mla {
 
-constexpr int kRowSt = 608;  // LDS row stride: 576 bytes + 32 of padding (38 chunk positions of 16 bytes)
-
-// 16-byte chunks of row r are XOR-swizzled by (r >> 2) & 7, which keeps the K
-// fragment reads (ds_read_b128) and the V^T transpose reads
-// (ds_read_b64_tr_b8) near their bank-conflict floor.
-__device__ __forceinline__ int g128_key(int r) { return (r >> 2) & 7; }
-// LDS chunk position (0..35) of logical chunk c of row r; an involution
-__device__ __forceinline__ int g128_pos(int r, int c) {
-  const int x = g128_key(r);
-  return c < 32 ? (c ^ x) : 32 + ((c - 32) ^ (x & 3));
-}
+constexpr int kRowSt = 576;           // LDS row stride: rows are not padded
+constexpr int kRowCh = kRowSt / 16;  // 16-byte chunks of a row
+// Chunk c of row r lies at position c ^ row_key(r) of the row.  The 144-dword
+// stride moves a row 16 banks, so the four rows r & 3 and the four keys cover
+// the 64 banks: neither the K fragment reads (ds_read_b128, 16 rows at one chunk)
+// nor the V^T transpose reads (ds_read_b64_tr_b8) conflict, no DMA lane is spent
+// on padding, and a fragment's address is one register plus constants (the key
+// moves only the chunk's low two bits, and rows 16 apart share it).
+__device__ __forceinline__ int row_key(int r) { return (r >> 2) & 3; }
 
 // v_permlane32_swap of x with itself: each lane ends with its own value and
 // its partner's (lane +- 32)
