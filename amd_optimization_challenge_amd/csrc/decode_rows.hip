@@ -16,8 +16,10 @@
 // Waves 0-3 score tile t while waves 4-7 run the PV of tile t - 1: as four waves
 // doing one after the other, a tile took its whole chain (fragment reads, nine
 // MFMAs, softmax, exchange, sixteen MFMAs), about 2.3 us; side by side 1.2, and
-// 256 x 1024 keys x 4 rows is gathered at 6.1 TB/s.  The 32 ragged sequences take
-// 16 us of decode instead of 48, the call 33.3-35.4 instead of 58.0.
+// 64 keys more of 256 sequences x 4 rows cost what their gather does (6.1 TB/s).
+// The 32 ragged sequences take 24-26 us of decode instead of 48, the call 33.3-35.4
+// instead of 58.0; a third of the rest is start-up (Q of 64 columns quantized, 2 us;
+// the plan, slots and first rows, 4) and 64 KiB of output per item.
 //   Scoring wave w: token half w & 1, column half w >> 1, nine 32x32x64 MFMAs
 // (S^T = K . Q^T, Q^T of its 32 columns in 72 registers).  A lane's 16 scores
 // are one column's, and the tokens its bytes of the PV operand hold, so P' goes
