@@ -165,6 +165,18 @@ struct H16 {
   static constexpr int LDS = OFF_VOTE + 16;
   static_assert(BLOCKS_PER_CU == 1 || LDS <= 80 * 1024, "two work-groups per CU");
 };
+// bf16 PV: up to this magnitude a head's reference lies within 1 of the score it was
+// taken from, so a fused s c - m_ref finds the item's largest score at most 2 above
+// it and the second pass stands.  Past 2^31 half an ulp of the reference exceeds
+// kRebase: fused, no pass would ever stand.  There the product is rounded first,
+// as the reference was, and the maximum kept is the score's own (its distance
+// from a far reference would lose it).  A wave-uniform branch; the fused form saves
+// 4 VALU of 190 per wave and tile.
+constexpr float kFarRef = 16777216.0f;
+// bf16 PV: the reference of a head whose scores are all -inf so far; far, and below
+// any finite score, which starts the next pass (-inf would make every difference
+// NaN or inf).
+constexpr float kNoScoreRef = -3.0e38f;
 constexpr int kVScaleSpan = 31;  // fp4 V: P' = P 2^(e - E_ref) <= 2^(96 + 31) stays finite in bf16
 
 
@@ -587,8 +599,10 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
   float m_ref = 0.f, m_seen = neg_inf(), l_part = 0.f;
   bool have_ref = false;
   int e_ref = 127, e_seen = 0;  // fp4 V: reference and running max of the V block exponents
-  // (m_seen: fp8 V the wave's ceil max of a head, bf16 PV the lane's
-  // score max above m_ref)
+  // (m_seen: fp8 V the wave's ceil max of a head, bf16 PV the lane's score max
+  // above m_ref, or the score max itself while far_ref)
+  // bf16 PV: some head's reference lies past kFarRef (the same in every wave)
+  bool far_ref = false;
 
   auto prologue = [&](bool slots_issued, bool quant) __attribute__((always_inline)) {
     if (!slots_issued) {
@@ -615,7 +629,7 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
   // the old reference, V block exponents), over the lanes of a head and the waves
   auto set_refs = [&]() __attribute__((always_inline)) {
     float mx = fmaxf(m_seen, shfl_xor_f(m_seen, 16));
-    mx = __builtin_ceilf(m_ref + fmaxf(mx, shfl_xor_f(mx, 32)));
+    mx = __builtin_ceilf((far_ref ? 0.f : m_ref) + fmaxf(mx, shfl_xor_f(mx, 32)));
     m_seen = neg_inf();
     int* ex = reinterpret_cast<int*>(smem + C::OFF_E);
     const int e_w = C::VB16 ? wave_max(e_seen) : 0;
@@ -623,6 +637,8 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
     if (C::VB16 && lane == 0) ex[w] = e_w;
     lds_barrier();
     m_ref = fmaxf(fmaxf(xch[l16], xch[16 + l16]), fmaxf(xch[32 + l16], xch[48 + l16]));
+    if (m_ref == neg_inf()) m_ref = kNoScoreRef;
+    far_ref = __any(fabsf(m_ref) > kFarRef);
     if constexpr (C::VB16) e_ref = max(max(ex[0], ex[1]), max(ex[2], ex[3]));
   };
   // fp4 V: the wave's exponent steps of one tile, from its e8m0 dword plane
@@ -733,7 +749,17 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
         float pw[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) pw[r] = __builtin_fmaf(s[r], c, -m_ref);
-        m_seen = fmaxf(fmaxf(m_seen, fmaxf(pw[0], pw[1])), fmaxf(pw[2], pw[3]));
+        if (far_ref) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            float sc = s[r] * c;
+            asm volatile("" : "+v"(sc));  // no fused multiply-subtract
+            m_seen = fmaxf(m_seen, sc);
+            pw[r] = sc - m_ref;
+          }
+        } else {
+          m_seen = fmaxf(fmaxf(m_seen, fmaxf(pw[0], pw[1])), fmaxf(pw[2], pw[3]));
+        }
 #pragma unroll
         for (int r = 0; r < 4; ++r) pw[r] = __builtin_amdgcn_exp2f(pw[r]);
         if (nval < kTile) {
@@ -905,7 +931,7 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
     if constexpr (C::PB) {
       // a score or V block exponent too far above its reference anywhere in
       // the pass: run the item again from the maxima of the whole item
-      const bool over = ntiles > 0 && (__any(m_seen > kRebase) ||
+      const bool over = ntiles > 0 && (__any(m_seen > (far_ref ? m_ref + kRebase : kRebase)) ||
                                        (C::VB16 && __any(e_seen > e_ref + kVScaleSpan)));
       if (lane == 0) vote[w] = over ? 1 : 0;
       lds_barrier();

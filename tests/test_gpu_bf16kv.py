@@ -111,3 +111,43 @@ def test_bf16_cache_refuses_128_heads(cuda):
     q, kv, indptr, idx = _case([64], 128, seed=1)
     with pytest.raises(_lib.MlaLibraryError):
         custom_kernel(_data(q, kv, indptr, idx, 0.1))
+
+
+@pytest.mark.parametrize("lens", [[200, 70], [700, 1]])
+@pytest.mark.parametrize("log2q", [12, 18, 24])
+def test_bf16_cache_huge_scores(cuda, lens, log2q):
+    """Scores of 2^28 to 2^41, where the references' own rounding passes the distance
+    a pass may leave: it ends, at the row of the largest score."""
+    print(f"bf16 kv huge scores {lens} 2^{log2q}", flush=True)
+    q, kv, indptr, idx = _case(lens, 16, seed=11)
+    q[...] = 0
+    q[..., 575] = 2.0 ** log2q
+    pos = torch.cat([torch.arange(L) for L in lens])
+    kv[idx.long(), 0, 575] = (2.0 ** 17 * (1 + (pos % 128) / 128) * torch.where(pos == 65, 4.0, 1.0)).to(torch.bfloat16)
+    got = custom_kernel(_data(q, kv, indptr, idx, 0.0712))
+    torch.cuda.synchronize()
+    got = got.float().cpu()
+    for b, L in enumerate(lens):
+        # one-hot: the next score is at least 2^17 log2 units below; P = 1, so the
+        # row comes out as it is, to one bf16 rounding
+        row = kv[idx[int(indptr[b]) + (65 if L > 65 else L - 1)].long(), 0, :512].float()
+        assert torch.all((got[b] - row).abs() <= 2.0 ** -7 * row.abs())
+
+
+@pytest.mark.parametrize("masked", [-3.3e38, -1e30])
+@pytest.mark.parametrize("first", [64, 100, 200])
+def test_bf16_cache_masked_first_tiles(cuda, first, masked):
+    """The first tokens masked through a rope dim (scores of -inf or -1e30), the others'
+    scores far below zero: their softmax, not the masked tokens'."""
+    print(f"bf16 kv masked {first} {masked}", flush=True)
+    q, kv, indptr, idx = _case([230], 16, seed=12)
+    q[..., 575] = 8.0
+    kv[:, 0, 575] = -500.0
+    kv[idx[:first].long(), 0, 575] = masked
+    sm = 1 / math.sqrt(576)
+    got = custom_kernel(_data(q, kv, indptr, idx, sm))
+    torch.cuda.synchronize()
+    live = idx[first:].long()
+    k = kv[live, 0].double()
+    ref = torch.softmax(q[0].double() @ k.T * sm, -1) @ k[:, :512]
+    assert_close(got[0].float().cpu().numpy(), ref.float().numpy())
