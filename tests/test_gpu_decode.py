@@ -119,6 +119,30 @@ def test_mxfp4_value_scale_growth(cuda, growth):
         assert_close(got[b] / s, ref[b] / s)
 
 
+@pytest.mark.parametrize("contiguous", [False, True])
+@pytest.mark.parametrize("log2k", [10, 22, 30])
+def test_mxfp4_huge_scores(cuda, log2k, contiguous):
+    """Scores up to 2^42, whose references round by more than a pass may leave above
+    them: the call ends, at the row of the one largest score."""
+    from oracle import mla_oracle as O
+
+    print(f"mxfp4 huge scores 2^{log2k}", flush=True)
+    lens = [200, 70, 700]
+    q, kv, indptr, idx, _, _ = host_case(lens, 16, "mxfp4", seed=31, permute=not contiguous)
+    q, kv = torch.zeros_like(q), kv.clone()
+    q[..., 575] = 2.0 ** 14
+    kv[:, 0, 544:575] = 0.0
+    kv[:, 0, 575] = 2.0 ** log2k
+    for b in range(len(lens)):  # past the first tile; the factor 4 is exact in any format
+        kv[idx[int(indptr[b]) + 66].long(), 0, 575] = 2.0 ** (log2k + 2)
+    case = case_from_tensors(q, kv, indptr, idx, "mxfp4")
+    data = device_data(q, kv, indptr, idx, case[5], "mxfp4", 0.0712, pass_indices=not contiguous)
+    got = custom_kernel(data)
+    torch.cuda.synchronize()
+    _, ref = O.reference_path(case[4], "mxfp4", case[5], indptr.numpy(), idx.numpy(), 0.0712)
+    assert_close(got.float().cpu().numpy(), ref)
+
+
 @pytest.mark.parametrize("heads,mode", [(16, "mxfp4"), (16, "mxfp4k_fp8v"), (128, "mxfp4k_fp8v")])
 def test_mxfp4_scale_row_stride(cuda, heads, mode):
     """The e8m0 scale rows may be padded (stride > 18, odd or even); every
