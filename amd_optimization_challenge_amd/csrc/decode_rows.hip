@@ -27,6 +27,9 @@
 //   PV wave: latent dims 128 (w - 4) .. +127 of all 64 columns, sixteen 32x32x64
 // MFMAs a tile with every K lane in use (two fp8 terms of P', V^T fragments shared
 // by both column halves); it also gathers the rows of tile t + 2, nine DMA windows.
+// The columns share a tile's V, so at the sequence's end a key that some of them
+// must not see is multiplied by their zero P': its NaN codes are read as 0 there (a
+// column that sees such a key has a NaN score from the same bytes, and stays NaN).
 // Two barriers a tile: (A) tile t landed, P'(t - 1) written, the stage of tile
 // t - 2 free; (B) P'(t - 1) in the PV waves' registers, so P'(t) may take its
 // place.  Most of the PV runs before B, beside the scores.
@@ -66,6 +69,12 @@ struct R64 {
   static_assert(STAGE % 4096 == 0 && COLS * kQKDim <= STAGE, "DMA windows, Q staging");
   static_assert(4 * COLS * OST <= OFF_SLOT && LDS <= 160 * 1024, "LDS");
 };
+
+// four e4m3 codes with the NaNs (0x7F, 0xFF) as 0
+__device__ __forceinline__ int nan_codes_to_zero(int x) {
+  const uint32_t n = (((uint32_t)x & 0x7F7F7F7Fu) + 0x01010101u) & 0x80808080u;  // bit 7 of a NaN's byte
+  return (int)((uint32_t)x & ~(n | (n - (n >> 7))));
+}
 
 template <bool IDX>
 __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams p) {
@@ -339,12 +348,17 @@ __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams 
           a1[e] = va[2 + e] + ((t - 1) & 3) * C::STAGE;
           asm volatile("" : "+v"(a0[e]), "+v"(a1[e]));
         }
+        const bool tail = t_beg + 64 * t > t_end - (qlen - 1);  // tile t - 1 holds keys that not every column sees
         auto pv = [&](auto et) __attribute__((always_inline)) {
           constexpr int e = decltype(et)::value;
           const uint32_t x0 = a0[e & 1] + 64 * (e >> 1), x1 = a1[e & 1] + 64 * (e >> 1);
           const v2i r0 = lds_read_tr8(x0), r1 = lds_read_tr8(x1);
           const v2i r2 = lds_read_tr8(x0 + C::TSTAGE), r3 = lds_read_tr8(x1 + C::TSTAGE);
-          const v8i vf = v8i{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
+          v8i vf = v8i{r0[0], r0[1], r1[0], r1[1], r2[0], r2[1], r3[0], r3[1]};
+          if (tail) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) vf[i] = nan_codes_to_zero(vf[i]);
+          }
 #pragma unroll
           for (int term = 0; term < 2; ++term)
 #pragma unroll

@@ -84,6 +84,31 @@ def test_second_pass_from_higher_references():
     _check(case, qb, qlen, 1 / np.sqrt(192), out, lse)
 
 
+@pytest.mark.parametrize("qlen", [2, 3, 4])
+@pytest.mark.parametrize("contiguous", [False, True])
+@pytest.mark.parametrize("back", [1, 2, 3])
+@pytest.mark.parametrize("dim", [100, 550])
+def test_nan_codes_stay_with_the_rows_that_see_them(qlen, contiguous, back, dim):
+    """A NaN code in one of a sequence's last keys (latent and rope dims; the masked
+    tail inside one tile, over two, and repeated past the item's end): the rows that
+    see the key are NaN throughout, the others as without it."""
+    lens = [70, 130, 5, 64, 65, 66, 192]
+    q = torch.randn(len(lens) * qlen, 16, 576, generator=torch.Generator().manual_seed(back)).to(torch.bfloat16)
+    case = host_case(lens, 16, "fp8", seed=5, permute=not contiguous)
+    _, kv, indptr, idx, _, caches = case
+    codes = caches["fp8_codes"].copy()
+    for b in range(len(lens)):
+        codes[int(idx[int(indptr[b + 1]) - back]), dim] = 0x7F if b % 2 else 0xFF
+    out, lse = _run((*case[:5], dict(caches, fp8_codes=codes)), q, qlen, 0.08, contiguous)
+    _, ref, ref_lse = O.reference_path(O.bf16_tensor_bits(q), "fp8", caches, indptr.numpy(), idx.numpy(), 0.08,
+                                       q_seq_len=qlen, return_lse=True)
+    sees = np.array([i >= qlen - back for _ in lens for i in range(qlen)])  # row i ends qlen - 1 - i keys early
+    assert out[torch.from_numpy(sees).to(DEV)].isnan().all()
+    assert_close(out.float().cpu().numpy()[~sees], ref[~sees])
+    got, want = lse.cpu().numpy()[~sees], ref_lse[~sees]
+    assert np.all(np.abs(got - want) <= 1e-2 + 1e-2 * np.abs(want))
+
+
 @pytest.mark.parametrize("qlen", [2, 4])
 def test_workspace_sizes(qlen):
     """The size of mla_workspace_bytes is accepted (fewer pieces), a byte less refused."""
