@@ -259,12 +259,15 @@ __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams 
             have_ref = true;
           }
           m_seen = fmaxf(m_seen, mx);
-          overflow = overflow || mx > m_ref + kRebaseR;
+          overflow = overflow || mx - m_ref > kRebaseR;  // (m_ref + kRebaseR would round at scores past 2^30)
           // the exponent: clamped (a flagged pass is run again), and finite where
           // the half is masked (its P' is 0 whatever the exponent)
           mx = fminf(fmaxf(mx, m_ref - 160.f), m_ref + kRebaseR);
-          e8 = min(max((int)(mx - m_ref) - 8 + 127, 0), 254);
-          const float sh = 8.f - mx;
+          // P' = 2^(s - mx + up): up = 8 uses the fp8 range; none where it would
+          // round (scores past 2^26 lie 8 apart or more: P' is 1, 2^-8 or next to 0)
+          const float up = fabsf(mx) < 67108864.f ? 8.f : 0.f;
+          e8 = min(max((int)(mx - m_ref - up) + 127, 0), 254);
+          const float sh = up - mx;
           float ps[4] = {0.f, 0.f, 0.f, 0.f};
           int2 q4[4];
 #pragma unroll
@@ -276,7 +279,7 @@ __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams 
             }
             q4[q] = split4(s[4 * q], s[4 * q + 1], s[4 * q + 2], s[4 * q + 3]);
           }
-          l_run = __builtin_fmaf((ps[0] + ps[1]) + (ps[2] + ps[3]), __builtin_amdgcn_exp2f(mx - m_ref - 8.f), l_run);
+          l_run = __builtin_fmaf((ps[0] + ps[1]) + (ps[2] + ps[3]), __builtin_amdgcn_exp2f(mx - m_ref - up), l_run);
           hi4 = make_int4(q4[0].x, q4[1].x, q4[2].x, q4[3].x);
           lo4 = make_int4(q4[0].y, q4[1].y, q4[2].y, q4[3].y);
         }

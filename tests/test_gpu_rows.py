@@ -84,6 +84,42 @@ def test_second_pass_from_higher_references():
     _check(case, qb, qlen, 1 / np.sqrt(192), out, lse)
 
 
+# sm_scale where the largest score is an odd multiple of 16 in [2^27, 2^28) log2 units:
+# half an ulp from its neighbours after adding the 8 that scales P to its fp8 range
+TIES = [0.048, 0.0635, 0.0765]
+
+
+def _log2_score(q_code, kv_code, qs, kvs, sm):
+    c = np.float32(qs) * np.float32(kvs) * np.float32(sm) * np.float32(1.4426950408889634)
+    return np.float32(q_code * kv_code) * c
+
+
+@pytest.mark.parametrize("contiguous", [False, True])
+@pytest.mark.parametrize("log2k,sm", [(15, s) for s in TIES] + [(10, 0.0712), (16, 0.0712), (18, 0.0712), (30, 0.0712)])
+def test_huge_scores(log2k, sm, contiguous):
+    """One largest score a sequence, up to 2^43: each row is that key's value."""
+    lens, qlen = [200, 70, 700], 3
+    _, kv, indptr, idx, _, _ = host_case(lens, 16, "fp8", seed=31, permute=not contiguous)
+    q, kv = torch.zeros(len(lens) * qlen, 16, 576, dtype=torch.bfloat16), kv.clone()
+    q[..., 575] = 2.0 ** 14
+    kv[:, 0, 544:575] = 0.0
+    kv[:, 0, 575] = 2.0 ** log2k
+    for b in range(len(lens)):  # past the first tile; the factor 4 is exact in e4m3
+        kv[idx[int(indptr[b]) + 66].long(), 0, 575] = 2.0 ** (log2k + 2)
+    kv[:, 0, :512] *= 2.0 ** (log2k - 1)
+    case = case_from_tensors(q[:3], kv, indptr, idx, "fp8")
+    _, qs = O.quantize_fp8_per_tensor(O.bf16_tensor_bits(q))
+    top = _log2_score(448, 448, qs, case[5]["fp8_scale"], sm)
+    if sm in TIES:
+        assert 2 ** 27 <= np.ceil(top) < 2 ** 28 and np.ceil(top) // 16 % 2 == 1, top
+    out, lse = _run(case, q, qlen, sm, contiguous)
+    _, ref, ref_lse = O.reference_path(O.bf16_tensor_bits(q), "fp8", case[5], indptr.numpy(), idx.numpy(), sm,
+                                       q_seq_len=qlen, return_lse=True)
+    got, unit = out.float().cpu().numpy(), 2.0 ** (log2k - 1)
+    assert_close(got / unit, ref / unit)
+    assert np.allclose(lse.cpu().numpy(), ref_lse, rtol=1e-2)
+
+
 @pytest.mark.parametrize("qlen", [2, 3, 4])
 @pytest.mark.parametrize("contiguous", [False, True])
 @pytest.mark.parametrize("back", [1, 2, 3])
