@@ -50,6 +50,10 @@ namespace {
 constexpr float kLog2eR = 1.4426950408889634f;
 constexpr float kLn2R = 0.6931471805599453f;
 constexpr float kRebaseR = 96.0f;
+// The reference of a column whose scores are all -inf so far (or that sees no key):
+// below any finite score, which starts the second pass; -inf itself would make the
+// differences NaN.
+constexpr float kNoScoreR = -3.0e38f;
 
 struct R64 {
   static constexpr int COLS = 64;
@@ -255,7 +259,7 @@ __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams 
             if (hh == 0) xch[C::COLS * th + col] = mx;
             lds_barrier();
             m_ref = fmaxf(xch[col], xch[C::COLS + col]);
-            if (m_ref == -__builtin_inff()) m_ref = 0.f;
+            m_ref = fmaxf(m_ref, kNoScoreR);
             have_ref = true;
           }
           m_seen = fmaxf(m_seen, mx);
@@ -298,7 +302,7 @@ __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams 
       lds_barrier();
       if (__builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(smem + C::OFF_VOTE)) == 0) break;
       m_ref = fmaxf(xch[col], xch[C::COLS + col]);
-      if (m_ref == -__builtin_inff()) m_ref = 0.f;
+      m_ref = fmaxf(m_ref, kNoScoreR);
       overflow = false;
       l_run = 0.f;
 #pragma unroll

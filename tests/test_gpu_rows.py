@@ -120,6 +120,28 @@ def test_huge_scores(log2k, sm, contiguous):
     assert np.allclose(lse.cpu().numpy(), ref_lse, rtol=1e-2)
 
 
+@pytest.mark.parametrize("contiguous", [False, True])
+def test_first_tile_of_minus_infinity(contiguous):
+    """Scores of a piece's first tile that overflow to -inf, finite ones after it: the
+    row is the mean of the finite keys' values."""
+    lens, qlen = [120, 100, 77], 3
+    _, kv, indptr, idx, _, _ = host_case(lens, 16, "fp8", seed=33, permute=not contiguous)
+    q, kv = torch.zeros(len(lens) * qlen, 16, 576, dtype=torch.bfloat16), kv.clone()
+    q[..., 575] = 2.0 ** 104
+    kv[:, 0, 512:575] = 0.0
+    kv[:, 0, :512] *= 2.0 ** 26
+    for b in range(len(lens)):  # a sequence is one piece of two tiles
+        slots = idx[int(indptr[b]):int(indptr[b + 1])].long()
+        kv[slots[:64], 0, 575] = -(2.0 ** 30)
+        kv[slots[64:], 0, 575] = -(2.0 ** 20)
+    case = case_from_tensors(q[:3], kv, indptr, idx, "fp8")
+    out, lse = _run(case, q, qlen, 0.0712, contiguous)
+    _, ref = O.reference_path(O.bf16_tensor_bits(q), "fp8", case[5], indptr.numpy(), idx.numpy(), 0.0712,
+                              q_seq_len=qlen)
+    assert np.isfinite(ref).all() and lse.isfinite().all()
+    assert_close(out.float().cpu().numpy() / 2.0 ** 26, ref / 2.0 ** 26)
+
+
 @pytest.mark.parametrize("qlen", [2, 3, 4])
 @pytest.mark.parametrize("contiguous", [False, True])
 @pytest.mark.parametrize("back", [1, 2, 3])
