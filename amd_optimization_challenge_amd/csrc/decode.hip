@@ -173,7 +173,7 @@ struct H16 {
 // from a far reference would lose it).  A wave-uniform branch; the fused form saves
 // 4 VALU of 190 per wave and tile.
 constexpr float kFarRef = 16777216.0f;
-// bf16 PV: the reference of a head whose scores are all -inf so far; far, and below
+// The reference of a head whose scores are all -inf so far; (bf16 PV) far, and below
 // any finite score, which starts the next pass (-inf would make every difference
 // NaN or inf).
 constexpr float kNoScoreRef = -3.0e38f;
@@ -792,6 +792,7 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
           if (g == 0) xch[16 * w + l16] = m_w;
           lds_barrier();
           m_ref = fmaxf(fmaxf(xch[l16], xch[16 + l16]), fmaxf(xch[32 + l16], xch[48 + l16]));
+          m_ref = fmaxf(m_ref, kNoScoreRef);
           have_ref = true;
         }
         const bool over = __any(m_w > m_ref + kRebase);
@@ -946,6 +947,7 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
       if (g == 0) xch[16 * w + l16] = m_seen;
       lds_barrier();
       m_ref = fmaxf(fmaxf(xch[l16], xch[16 + l16]), fmaxf(xch[32 + l16], xch[48 + l16]));
+      m_ref = fmaxf(m_ref, kNoScoreRef);
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) o[i] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -1027,15 +1029,16 @@ __global__ __launch_bounds__(256 * PG) void combine_kernel(const DecodeParams p)
     float mb = M;
 #pragma unroll
     for (int j = 0; j < 8; ++j) mb = fmaxf(mb, ls[j]);
-    if (mb == neg_inf()) continue;  // every piece so far is empty
-    const float r = M == neg_inf() ? 0.f : exp2f(M - mb);
+    // every piece so far is empty, or NaN (lse -inf too): weights 0, which keep the NaN
+    const float m0 = mb == neg_inf() ? 0.f : mb;
+    const float r = exp2f(M - m0);
     wsum *= r;
 #pragma unroll
     for (int i = 0; i < 8; ++i) acc[i] *= r;
     M = mb;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      const float wg = exp2f(ls[j] - M);  // 0 for padding slots (lse -inf)
+      const float wg = exp2f(ls[j] - m0);  // 0 for padding slots (lse -inf)
       wsum += wg;
       const uint32_t wv[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
 #pragma unroll
@@ -1058,18 +1061,17 @@ __global__ __launch_bounds__(256 * PG) void combine_kernel(const DecodeParams p)
     float m = M;
 #pragma unroll
     for (int g = 0; g < PG - 1; ++g) m = fmaxf(m, part[g][0][tid]);
-    if (m != neg_inf()) {
-      const float r = exp2f(M - m);  // 0 for a group that found only empty pieces
-      wsum *= r;
+    const float m0 = m == neg_inf() ? 0.f : m;
+    const float r = exp2f(M - m0);  // 0 for a group that found only empty (or NaN) pieces
+    wsum *= r;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) acc[i] *= r;
+    for (int i = 0; i < 8; ++i) acc[i] *= r;
 #pragma unroll
-      for (int g = 0; g < PG - 1; ++g) {
-        const float rg = exp2f(part[g][0][tid] - m);
-        wsum += rg * part[g][1][tid];
+    for (int g = 0; g < PG - 1; ++g) {
+      const float rg = exp2f(part[g][0][tid] - m0);
+      wsum += rg * part[g][1][tid];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) acc[i] += rg * part[g][2 + i][tid];
-      }
+      for (int i = 0; i < 8; ++i) acc[i] += rg * part[g][2 + i][tid];
     }
     M = m;
   }
