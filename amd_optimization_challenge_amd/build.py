@@ -24,11 +24,16 @@ SOURCES = ["quant.hip", "decode.hip", "decode_h128.hip", "decode_rows.hip", "nei
 ARCH = os.environ.get("MLA_OFFLOAD_ARCH", "gfx950")
 
 # -packed-fp32-ops: keep the compiler from forming v_pk_{add,mul,fma}_f32
+# -fno-strict-aliasing: the kernels write LDS as one type and read it as another
+# (16-bit exponent steps as 16-byte vectors), not always with a barrier between;
+# type-based alias analysis could swap the two.  The code is the same with and
+# without it, instruction for instruction.
 CFLAGS = [
     "-O3",
     "-std=c++17",
     f"--offload-arch={ARCH}",
     "-fPIC",
+    "-fno-strict-aliasing",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wall",
     "-Wno-unused-function",

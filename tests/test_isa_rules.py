@@ -24,6 +24,7 @@ one wait state (gfx9-family rule for an SALU write of M0 read by an LDS DMA).
    metadata: private segment size and VGPR spill count 0), except the a16w8
    variant of the 16-head kernel (two fp8 terms of Q, 80 registers, at two
    work-groups per CU), which is on no benchmarked route.
+6. No type-based alias analysis: LDS is written as one type and read as another.
 
 ``python tests/test_isa_rules.py --resources`` prints the per-kernel register,
 LDS and scratch figures of the built library as a markdown table.
@@ -305,6 +306,29 @@ def test_no_scratch_in_the_operator_kernels(tmp_path):
                 bad.append(f"{obj} {k['name']}: {k['scratch']} B scratch, {k['vgpr_spill']} VGPRs spilled")
     assert seen >= 20, seen
     assert not bad, "\n".join(bad)
+
+
+def test_lds_accesses_of_different_types_stay_in_order(tmp_path):
+    """Device code built with the library's flags carries no type-based alias tags,
+    so a store of one type and a load of another to the same bytes keep their order."""
+    sys.path.insert(0, ROOT)
+    from amd_optimization_challenge_amd import build
+
+    try:
+        cc = build.hipcc()
+    except RuntimeError:
+        pytest.skip("hipcc not found")
+    src = tmp_path / "alias.hip"
+    src.write_text("#include <hip/hip_runtime.h>\n#include <stdint.h>\n"
+                   "__global__ void k(uint4* o, uint16_t v) {\n"
+                   "  __shared__ __attribute__((aligned(16))) uint8_t m[1024];\n"
+                   "  reinterpret_cast<uint16_t*>(m)[threadIdx.x] = v;\n"
+                   "  o[threadIdx.x] = reinterpret_cast<uint4*>(m)[threadIdx.x & 7];\n}\n")
+    ir = tmp_path / "alias.ll"
+    subprocess.run([cc, *build.CFLAGS, "--cuda-device-only", "-S", "-emit-llvm", str(src), "-o", str(ir)], check=True,
+                   capture_output=True)
+    text = ir.read_text()
+    assert "store i16" in text and "!tbaa" not in text
 
 
 def resources_markdown():
