@@ -290,17 +290,45 @@ def combine(batch: int, num_heads: int, ws: torch.Tensor, out: torch.Tensor, lse
     _call("mla_combine", ws.device, batch, num_heads, _ptr(ws), ws.numel(), _ptr(out), _ptr(lse))
 
 
-def _rows_together(q_seq_len: int, num_heads: int, mode: int, tokens: int) -> bool:
+def _rows_together(q_seq_len: int, num_heads: int, mode: int, tokens: int, sequences: int, indexed: bool) -> bool:
     """The causal rows of a sequence as one pass over its cache
-    (``mla_decode_fwd_rows``) instead of a pass per row.  It saves q_seq_len - 1
-    gathers of at most ``tokens`` cached rows (580 bytes at about 5.4 TB/s) and
-    costs about 4 us of longer prologue and finish per work-group (64 columns,
-    one work-group per CU), so it pays from (q_seq_len - 1) x tokens = 2^15.
-    Whole calls on MI355X, a pass per row against this: 60 x 160 tokens x 4 rows
-    19.7 / 23.7 us and 32 x 800 x 2 22.9 / 23.3 (below the line), 100 x 200 x 3
-    31.6 / 25.9, 300 x 40 x 4 38.2 / 34.1 and 32 of 512 to 8192 x 4 58.0 / 33.3
-    (above it)."""
-    return num_heads == 16 and mode == 0 and 2 <= q_seq_len <= 4 and (q_seq_len - 1) * tokens >= 1 << 15
+    (``mla_decode_fwd_rows``) instead of a pass per row.  It saves
+    extra = (q_seq_len - 1) x ``tokens`` gathered rows and costs about 4 us of longer
+    prologue and finish per work-group (64 columns), on one work-group per CU
+    where the passes per row run two.  So it pays once the extra gathers outweigh
+    that, and not where the passes per row run side by side anyway (few
+    sequences).  Whole calls on MI355X over caches read in turn, a pass per row
+    against this, us:
+
+    * many rows over scattered slots, from extra = 2^15 (192 sequences x 170 tokens
+      x 2 rows 32.5 / 20.3; 256 x 128 x 4 40.9 / 25.4; 60 x 160 x 4, below, 19.7 /
+      23.7; 257 to 383 sequences take two rounds of work-groups here, as do 384
+      and more, which pays at three rows)
+    * up to 11 contiguous rows: never, a row's 32 pieces leave CUs for the others
+      (1 x 32768 x 4 34.7 / 41.2, 4 x 8192 x 2 20.9 / 23.4; 3 x 21845 x 4 41.2 / 37.0)
+    * one or two sequences over slots: from 2^18 tokens (1 x 32768 x 4 33.6 / 52.8,
+      2 x 16384 x 4 31.4 / 40.6; 2 x 131072 x 3 100.8 / 62.0)
+    * more than 256 sequences: from 2^17 tokens over slots, 3 x 2^16 contiguous (300 x
+      218 x 3 contiguous 44.7 / 57.4; 300 x 873 x 4 128.9 / 86.5)
+    * 24 to 255 sequences: from extra = 3 x 2^15 (32 x 1024 x 2 19.6 / 20.8; 32 of 512
+      to 8192 x 4 58.0 / 33.3); others from 2^17 (8 x 4096 x 4 24.4 / 28.8, 16 x
+      4096 x 4 35.0 / 29.4)
+
+    Over 3330 calls (1 to 1000 sequences, 4096 to 10^6 tokens) a pass per row is
+    more than 3 % faster in 12 of those the rule takes, 15 % at most."""
+    if num_heads != 16 or mode != 0 or not 2 <= q_seq_len <= 4:
+        return False
+    extra, rows = (q_seq_len - 1) * tokens, q_seq_len * sequences
+    if indexed:
+        if extra >= 1 << 15 and rows >= 384 and (sequences <= 256 or sequences >= 384 and q_seq_len > 2):
+            return True
+        if sequences < 3:
+            return tokens >= 1 << 18
+    elif rows < 12:
+        return False
+    if sequences > 256:
+        return tokens >= (1 << 17 if indexed else 3 << 16)
+    return extra >= (3 << 15 if 24 <= sequences < 256 else 1 << 17)
 
 
 def decode_fwd(q, kv_data, kv_indptr, kv_indices, sm_scale, kv_mode="fp8", out=None, ws=None, q_seq_len=1,
@@ -341,7 +369,8 @@ def decode_fwd(q, kv_data, kv_indptr, kv_indices, sm_scale, kv_mode="fp8", out=N
     mode = kv_mode_id(kv_mode)
     k, ks, ksc, kss, v, vs, sc = _kv_args(mode, kv_data)
     rows = q_dtype == "fp8" and _rows_together(q_seq_len, num_heads, mode,
-                                               k.shape[0] if kv_indices is None else kv_indices.numel())
+                                               k.shape[0] if kv_indices is None else kv_indices.numel(),
+                                               batch // q_seq_len, kv_indices is not None)
     if ws is None:
         ws = _ws_cache.get((batch, num_heads, mode, q.device, q_seq_len if rows else 1))
         if ws is None:

@@ -214,8 +214,9 @@ int mla_decode_fwd(const void* q_bf16, const void* k_cache, int64_t k_row_stride
 /*
  * mla_decode_fwd for the causal rows of multi-token sequences (16 heads, fp8
  * cache, q_seq_len 2 to 4): the rows of a sequence share one pass over its
- * cache instead of a pass each.  Same arguments and result; it pays once
- * (q_seq_len - 1) x cached tokens is above about 32768 (ops.decode_fwd's rule).
+ * cache instead of a pass each.  Same arguments and result.  It pays for 24 to 255
+ * sequences once (q_seq_len - 1) x cached tokens is above about 98304 and later
+ * for fewer or more (ops.decode_fwd's rule has the lines and both sides' times).
  * Workspace: mla_workspace_bytes_qlen, or at least mla_workspace_bytes.
  */
 int mla_decode_fwd_rows(const void* q_bf16, const void* k_cache, int64_t k_row_stride, const void* k_scales,
