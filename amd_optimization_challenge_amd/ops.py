@@ -332,7 +332,7 @@ def _rows_together(q_seq_len: int, num_heads: int, mode: int, tokens: int, seque
 
 
 def decode_fwd(q, kv_data, kv_indptr, kv_indices, sm_scale, kv_mode="fp8", out=None, ws=None, q_seq_len=1,
-               return_lse=False, page_size=1, kv_last_page_lens=None, q_dtype="fp8", lse=None):
+               return_lse=False, page_size=1, kv_last_page_lens=None, q_dtype="fp8", lse=None, kv_seq_len=None):
     """Whole operator: FP8-quantize q, plan, decode, combine.
 
     q: bf16 [rows, H, 576], rows = sequences x q_seq_len (row i of a sequence
@@ -347,9 +347,12 @@ def decode_fwd(q, kv_data, kv_indptr, kv_indices, sm_scale, kv_mode="fp8", out=N
     quantized per head row inside the decode, which for up to 256 query rows
     also plans its own work (two launches per call).  q_dtype "fp8" with 16
     heads, the fp8 cache, q_seq_len 2 to 4 and enough cached tokens runs a
-    sequence's rows together (``_rows_together``).  ``out`` (bf16 [rows, H,
-    512]) and ``lse`` (f32 [rows, H], with ``return_lse``) may be passed in;
-    each is allocated here only when it is not.
+    sequence's rows together (``_rows_together``).  The cached tokens are counted
+    on the host, as the rows of a contiguous cache or the entries of kv_indices;
+    where those have room to spare, ``kv_seq_len`` (the longest sequence, in tokens)
+    bounds them: it only chooses the route.  ``out`` (bf16 [rows, H, 512])
+    and ``lse`` (f32 [rows, H], with ``return_lse``) may be passed in; each is
+    allocated here only when it is not.
     """
     if int(page_size) != 1:
         if kv_indices is None or kv_last_page_lens is None:
@@ -368,9 +371,13 @@ def decode_fwd(q, kv_data, kv_indptr, kv_indices, sm_scale, kv_mode="fp8", out=N
                          f"entries do not fit (need rows = sequences x q_seq_len, indptr = sequences + 1)")
     mode = kv_mode_id(kv_mode)
     k, ks, ksc, kss, v, vs, sc = _kv_args(mode, kv_data)
-    rows = q_dtype == "fp8" and _rows_together(q_seq_len, num_heads, mode,
-                                               k.shape[0] if kv_indices is None else kv_indices.numel(),
-                                               batch // q_seq_len, kv_indices is not None)
+    rows = False
+    if q_dtype == "fp8" and q_seq_len > 1:
+        seqs = batch // q_seq_len
+        tokens = k.shape[0] if kv_indices is None else kv_indices.numel()
+        if kv_seq_len is not None and kv_seq_len > 0:
+            tokens = min(tokens, seqs * kv_seq_len)
+        rows = _rows_together(q_seq_len, num_heads, mode, tokens, seqs, kv_indices is not None)
     if ws is None:
         ws = _ws_cache.get((batch, num_heads, mode, q.device, q_seq_len if rows else 1))
         if ws is None:

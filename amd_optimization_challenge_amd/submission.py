@@ -15,6 +15,8 @@ is taken to be ``arange * q_seq_len`` as generate_input makes it, :330), and
 a paged cache the way AITER's mla_decode_fwd does (aiter_mla.py:149-175): the
 caches shaped [pages, page_size, 1, row], ``kv_indptr`` over pages,
 ``config["kv_indices"]`` the page ids and ``config["kv_last_page_lens"]``.
+``config["kv_seq_len"]`` (the longest sequence) bounds the cached tokens by which
+a multi-token call's route is chosen; the result does not depend on it.
 ``config["q_dtype"] = "bf16"`` takes the reference's a16w8 route (bf16 Q, fp8
 cache, 16 heads; TASK/reference.py:55-58 Q_DTYPE) instead of a8w8.
 ``config["kv_mode"] = "auto"`` picks the cache by speed, as the reference's
@@ -93,9 +95,10 @@ def custom_kernel(data: input_t) -> output_t:
     if qo_indptr is not None and qo_indptr.numel() != kv_indptr.numel():
         raise ValueError("qo_indptr and kv_indptr must both have batch + 1 entries")
     page_size = int(config.get("page_size", 1))
+    kv_seq_len = config.get("kv_seq_len")  # the longest sequence: bounds the tokens where the cache has room to spare
     return_lse = bool(config.get("return_lse", False))
     out, lse = _outputs(q.shape[0], num_heads, q.device, return_lse)
     return ops.decode_fwd(q, kv_data, kv_indptr, kv_indices, sm_scale, kv_mode, out=out, q_seq_len=q_seq_len,
                           return_lse=return_lse, page_size=page_size,
                           kv_last_page_lens=config.get("kv_last_page_lens"),
-                          q_dtype=q_dtype, lse=lse)
+                          q_dtype=q_dtype, lse=lse, kv_seq_len=kv_seq_len if isinstance(kv_seq_len, int) else None)

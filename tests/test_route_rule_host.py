@@ -1,8 +1,9 @@
 """Which calls run a sequence's causal rows together (ops._rows_together): both sides
 of every line of the rule, and calls measured to be faster one way or the other."""
 import pytest
+import torch
 
-from amd_optimization_challenge_amd import ops
+from amd_optimization_challenge_amd import ops, submission
 
 
 @pytest.mark.parametrize("qlen,seqs,tokens,indexed", [
@@ -31,3 +32,25 @@ def test_rows_together(qlen, seqs, tokens, indexed):
 @pytest.mark.parametrize("qlen,heads,mode", [(1, 16, 0), (5, 16, 0), (4, 128, 0), (4, 16, 1), (4, 16, 2), (4, 16, 3)])
 def test_what_the_kernel_does_not_take(qlen, heads, mode):
     assert not ops._rows_together(qlen, heads, mode, 1 << 30, 32, True)
+
+
+@pytest.mark.parametrize("kv_seq_len,tokens,indexed,together", [
+    (160, 9600, True, False), (160, 1 << 17, True, False), (160, 1 << 17, False, False),  # room to spare
+    (None, 9600, True, False), (None, 1 << 17, True, True), (0, 1 << 17, True, True), (4000, 1 << 17, True, True),
+    (4000, 1 << 17, False, True)])
+def test_tokens_are_bounded_by_the_longest_sequence(monkeypatch, kv_seq_len, tokens, indexed, together):
+    """Sixty sequences x 4 rows through custom_kernel: a cache or an index list larger
+    than the sequences fill does not take a short call to the route of a long one."""
+    called = []
+    monkeypatch.setattr(ops, "_require_cuda", lambda *a: None)
+    monkeypatch.setattr(ops, "workspace", lambda *a: torch.empty(0, dtype=torch.uint8))
+    monkeypatch.setattr(ops, "_call", lambda name, *a: called.append(name))
+    monkeypatch.setattr(submission, "_out_cache", {})
+    monkeypatch.setattr(ops, "_ws_cache", {})
+    kv = {"fp8": (torch.empty((1, 1, 576), dtype=torch.uint8).expand(tokens, 1, 576), torch.ones(1))}
+    cfg = dict(q_seq_len=4, kv_indices=torch.zeros(1, dtype=torch.int32).expand(tokens) if indexed else None)
+    if kv_seq_len is not None:
+        cfg["kv_seq_len"] = kv_seq_len
+    submission.custom_kernel((torch.zeros((240, 16, 576), dtype=torch.bfloat16), kv, None,
+                              torch.zeros(61, dtype=torch.int32), cfg))
+    assert called == ["mla_decode_fwd_rows" if together else "mla_decode_fwd"]
