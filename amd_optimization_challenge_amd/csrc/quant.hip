@@ -23,6 +23,12 @@ __device__ __forceinline__ void build_plan(const int32_t* __restrict__ kv_indptr
                                            int target_items, int min_chunk, int max_splits, int max_items,
                                            int32_t* __restrict__ plan);
 
+// NT: streaming loads, for an input well past the last-level cache (the quantizer
+// finds little of it there).  Both passes, default / streaming: 253 MB 107.8 / 117.1
+// us, 302 MB 133.8 / 138.8, 334 MB 153.2 / 155.5, 369 MB 179 / 175, 461 MB 225 / 218,
+// 604 MB 299 / 290.
+constexpr int64_t kAmaxStreamElems = 168LL << 20;
+template <bool NT>
 __global__ __launch_bounds__(256) void amax_kernel(const uint16_t* __restrict__ x, int64_t n,
                                                    uint32_t* __restrict__ partials, int nblocks,
                                                    const int32_t* __restrict__ kv_indptr,
@@ -52,13 +58,14 @@ __global__ __launch_bounds__(256) void amax_kernel(const uint16_t* __restrict__ 
   uint32_t m = 0;
   const int64_t nvec = n >> 3;
   const uint4* xv = reinterpret_cast<const uint4*>(x);
-  // Default cache policy: the quantizer reads the same values next, from the 256
-  // MB last-level cache where they fit.  Streaming loads here are faster by
+  // Default cache policy (!NT): the quantizer reads the same values next, from the
+  // 256 MB last-level cache where they fit.  Streaming loads here are faster by
   // themselves (151 MB: 26.8 us against 34.4) and cost the quantizer more (47.7
-  // against 39.8); at 38 MB 10.7 / 10.7 and 12.2 / 10.3.  Eight loads in flight
-  // per thread changed nothing at 151 MB and lost 2 us at 38.
+  // against 39.8); at 38 MB 10.7 / 10.7 and 12.2 / 10.3.  Past kAmaxStreamElems
+  // too little of the input is left there.  Eight loads in flight per thread
+  // changed nothing at 151 MB and lost 2 us at 38.
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < nvec; i += (int64_t)nblocks * 256) {
-    const uint4 v = xv[i];
+    const uint4 v = NT ? ldg16_nt(xv + i) : xv[i];
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -539,7 +546,8 @@ hipError_t launch_amax(const uint16_t* x, int64_t n, uint32_t* partials, int* nb
   const int nb = amax_blocks_for(n);
   *nblocks = nb;
   const int grid = nb + (plan != nullptr ? 1 : 0);
-  hipLaunchKernelGGL(amax_kernel, dim3(grid), dim3(256), 0, stream, x, n, partials, nb, kv_indptr,
+  const auto kernel = n > kAmaxStreamElems ? amax_kernel<true> : amax_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, stream, x, n, partials, nb, kv_indptr,
                      plan != nullptr ? kv_indices : nullptr, batch, qlen, target.items, target.min_chunk,
                      target.max_splits, max_items, plan);
   return hipGetLastError();

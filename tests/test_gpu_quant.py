@@ -85,3 +85,19 @@ def test_mxfp4_pack_golden_and_padded_scales(cuda):
     packed, scales = gpu_pack(d["x"], scale_cols=24)
     assert np.array_equal(packed, d["packed"])
     assert np.array_equal(scales[:, :18], d["scales"]) and np.all(scales[:, 18:] == 127)
+
+
+@pytest.mark.parametrize("extra", [0, 11])
+def test_streaming_amax_equals_the_cached_one(cuda, extra):
+    """Inputs past the streaming line of the amax pass (168 Mi values) give the codes
+    of their parts below it; the maximum is the last value."""
+    n = (168 << 20) + extra
+    x = torch.empty(n, dtype=torch.bfloat16, device=cuda)
+    x.normal_(generator=torch.Generator(device=cuda).manual_seed(extra))
+    x[-1] = -100.0
+    codes, scale = ops.quant_fp8_per_tensor(x)
+    half = n // 2
+    for part in (slice(0, half), slice(half, n)):
+        want, want_scale = ops.quant_fp8_per_tensor(torch.cat([x[part], x[-1:]]))
+        assert torch.equal(scale, want_scale)
+        assert torch.equal(codes.view(torch.uint8)[part], want.view(torch.uint8)[:-1])
