@@ -65,9 +65,9 @@ def test_sm_scale_is_honoured(cuda, heads, mode):
 
 @pytest.mark.parametrize("heads,mode", MODES)
 def test_wide_score_range(cuda, heads, mode):
-    """Scores that climb by ~100 (log2 units) per 64-token tile: far beyond the
-    fp8 range of P, so every tile needs its own offset (and, for H=128, the
-    accumulator reference restarts)."""
+    """Scores that climb by 25 log2 units per 64-token tile: beyond the fp8 range
+    of P, so every tile needs its own offset (items that run again from higher
+    references: test_gpu_second_pass.py)."""
     print(f"wide score range H={heads} mode={mode}", flush=True)
     g = torch.Generator().manual_seed(17)
     lens = [700, 130, 5]
@@ -92,10 +92,10 @@ def test_wide_score_range(cuda, heads, mode):
 def test_mxfp4_value_scale_growth(cuda, growth):
     """fp4 V (H = 16): the per-token MX block scales are folded into P relative
     to a per-item reference exponent.  Latent values that grow by 2^growth
-    over the sequence push later block exponents above it (45 and 90 exceed
-    the span a bf16 P' can carry, so the item restarts from a higher
-    reference); Q is zero on dims 0..511, so the scores stay ordinary while V
-    (and K's first 512 dims) change scale."""
+    over the sequence give its 128-token items different references, each with
+    later block exponents up to 17 above it (past 31 an item runs again:
+    test_gpu_second_pass.py); Q is zero on dims 0..511, so the scores stay
+    ordinary while V (and K's first 512 dims) change scale."""
     print(f"mxfp4 V scale growth 2^{growth}", flush=True)
     g = torch.Generator().manual_seed(23)
     lens = [700, 129, 64]
