@@ -18,12 +18,13 @@ s_nop N counts N + 1 wait states, every other instruction one.
 
 2. Every LDS-DMA (global_load_lds_*) follows the last write of M0 by at least
 one wait state (gfx9-family rule for an SALU write of M0 read by an LDS DMA).
-3. No scalar-memory stores, atomics or cache write-backs in any kernel.
+3. Every scalar-memory instruction (by its encoding) is a load, in any kernel.
 4. No packed-FP32 add/mul/fma (the build disables their formation).
 5. No decode, combine, quant or planner kernel spills to scratch (code-object
    metadata: private segment size and VGPR spill count 0), except the a16w8
-   variant of the 16-head kernel (two fp8 terms of Q, 80 registers, at two
-   work-groups per CU), which is on no benchmarked route.
+   variants of the 16-head kernel: two fp8 terms of Q take 80 registers at two
+   work-groups per CU, and 24 (kv_indices) and 68 bytes a lane of what is set up
+   once per item go to scratch.  They may not take more.
 6. No type-based alias analysis: LDS is written as one type and read as another.
 
 ``python tests/test_isa_rules.py --resources`` prints the per-kernel register,
@@ -214,7 +215,7 @@ def _objects(tmp_path):
             d = tmp_path / f[:-2]
             d.mkdir()
             try:
-                out[f] = parse(disassemble(os.path.join(BUILD, f), str(d)))
+                out[f] = disassemble(os.path.join(BUILD, f), str(d))
             except subprocess.CalledProcessError as e:
                 if b".hip_fatbin' not found" in (e.stderr or b""):
                     continue  # host code only
@@ -234,17 +235,32 @@ def m0_wait_violations(insns):
     return bad
 
 
-FORBIDDEN_SCALAR = ("s_store", "s_buffer_store", "s_scratch_store", "s_atomic", "s_buffer_atomic", "s_dcache_wb")
+# Scalar-memory instructions carry 110000 in the top six bits of their first dword.
+SMEM_ENCODING = 0b110000
+SMEM_LOADS = ("s_load_dword", "s_buffer_load_dword", "s_memtime")  # s_memtime: the cycle counter
+
+
+def smem_violations(text):
+    """Scalar-memory instructions of a disassembly that are not loads."""
+    bad = []
+    for line in text.splitlines():
+        m = INSN.match(line)
+        if m and int(m.group(4).split()[0], 16) >> 26 == SMEM_ENCODING and not m.group(1).startswith(SMEM_LOADS):
+            bad.append(f"{m.group(1)} {m.group(2)}")
+    return bad
+
+
 FORBIDDEN_PACKED = ("v_pk_add_f32", "v_pk_mul_f32", "v_pk_fma_f32")
 
 
 def test_code_object_rules(tmp_path):
     report = []
-    for obj, funcs in _objects(tmp_path).items():
-        for name, insns in funcs.items():
+    for obj, text in _objects(tmp_path).items():
+        report += [f"{obj}: {b}" for b in smem_violations(text)]
+        for name, insns in parse(text).items():
             report += [f"{obj} {name}: {b}" for b in m0_wait_violations(insns)]
             for _, mnem, args, _ in insns:
-                if mnem.startswith(FORBIDDEN_SCALAR) or mnem in FORBIDDEN_PACKED:
+                if mnem in FORBIDDEN_PACKED:
                     report.append(f"{obj} {name}: {mnem} {args}")
     assert not report, "\n".join(report[:20])
 
@@ -255,6 +271,14 @@ def test_m0_rule_checker():
     bad = [ok[0], ok[1], (8, "global_load_lds_dwordx4", "v[2:3], off", None)]
     assert not m0_wait_violations(ok)
     assert m0_wait_violations(bad)
+
+
+def test_scalar_memory_rule_checker():
+    load = "\ts_load_dwordx2 s[0:1], s[4:5], 0x8    // 000000001000: C0060002 00000008"
+    alu = "\ts_add_u32 s0, s1, s2                   // 000000001008: 80000201"
+    other = "\ts_anything s0, s[4:5], 0x8            // 00000000100C: C0420002 00000008"
+    assert not smem_violations("\n".join((load, alu)))
+    assert len(smem_violations("\n".join((load, alu, other)))) == 1
 
 
 def kernel_metadata(obj, tmp):
@@ -282,8 +306,9 @@ def kernel_metadata(obj, tmp):
     return out
 
 
-SCRATCH_CHECKED = ("decode.o", "decode_h128.o", "quant.o", "noalloc.o")
-A16W8 = re.compile(r"decode_h16_kernelILi0ELi0ELb[01]ELi2E")
+SCRATCH_CHECKED = ("decode.o", "decode_h128.o", "decode_rows.o", "quant.o", "noalloc.o")
+A16W8 = re.compile(r"decode_h16_kernelILi0ELi0ELb([01])ELi2E")
+A16W8_SCRATCH = {"0": 68, "1": 24}
 
 
 def test_no_scratch_in_the_operator_kernels(tmp_path):
@@ -300,11 +325,12 @@ def test_no_scratch_in_the_operator_kernels(tmp_path):
         d.mkdir()
         for k in kernel_metadata(path, str(d)) or []:
             seen += 1
-            if A16W8.search(k["name"]):
+            a16w8 = A16W8.search(k["name"])
+            if a16w8 and k["scratch"] <= A16W8_SCRATCH[a16w8.group(1)]:
                 continue
             if k["scratch"] or k["vgpr_spill"]:
                 bad.append(f"{obj} {k['name']}: {k['scratch']} B scratch, {k['vgpr_spill']} VGPRs spilled")
-    assert seen >= 20, seen
+    assert seen >= 22, seen
     assert not bad, "\n".join(bad)
 
 
