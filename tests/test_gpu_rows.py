@@ -1,8 +1,8 @@
 """The causal rows of a sequence as one work item (16 heads, fp8 cache, q_seq_len 2
 to 4) at the edges of its tiles: one-token to many-tile sequences, rows that see
-nothing, pieces whose end lies inside the last rows' masked tail, a second pass from
-higher references, more sequences than the planner sorts, and workspaces of both
-sizes; against the oracle."""
+nothing, pieces whose end lies inside the last rows' masked tail, scores and codes at
+the ends of their ranges, a captured graph, more sequences than the planner sorts,
+and workspaces of both sizes; against the oracle."""
 import ctypes
 
 import numpy as np
@@ -62,8 +62,9 @@ def test_more_sequences_than_the_planner_sorts():
     _check(case, q, 2, 0.08, out, lse)
 
 
-def test_second_pass_from_higher_references():
-    """Scores that climb by ~100 (log2 units) per tile: past the accumulators' range."""
+def test_scores_that_climb():
+    """Scores that climb by 25 log2 units per tile, past the fp8 range of P: every half
+    tile needs its own exponent (the second pass: test_gpu_second_pass.py)."""
     g = torch.Generator().manual_seed(17)
     lens, qlen = [700, 130, 5], 4
     T = sum(lens)
@@ -180,3 +181,37 @@ def test_workspace_sizes(qlen):
     _check(case, q, qlen, 0.08, out, lse)
     with pytest.raises(_lib.MlaLibraryError):
         _run(case, q, qlen, 0.08, ws=ws[:-256])
+
+
+def test_captured_calls_follow_their_inputs():
+    """The route in a graph, replayed with eager calls between: new queries and other
+    lengths in the same buffers give the eager call's bits each time."""
+    lens, qlen = [1500, 700, 64, 3], 4
+    case = host_case(lens, 16, "fp8", seed=8)
+    q, kv, indptr, idx, _, caches = case
+    _, kv_data, _, kv_indptr, cfg = device_data(q, kv, indptr, idx, caches, "fp8", 0.08)
+    g = torch.Generator(device=DEV).manual_seed(1)
+    q = torch.randn(16, 16, 576, device=DEV, generator=g).to(torch.bfloat16)
+    ws = torch.empty(ops.workspace_bytes(16, 16, "fp8", qlen), dtype=torch.uint8, device=DEV)
+    out = torch.empty(16, 16, 512, dtype=torch.bfloat16, device=DEV)
+    lse = torch.empty(16, 16, dtype=torch.float32, device=DEV)
+
+    def call(ws, out, lse):
+        ops.decode_fwd(q, kv_data, kv_indptr, cfg["kv_indices"], 0.08, "fp8", out=out, ws=ws, q_seq_len=qlen,
+                       return_lse=True, lse=lse)
+
+    call(ws, out, lse)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call(ws, out, lse)
+    for i, cut in enumerate([0, 100, 700, 1436]):  # the first sequence loses its last keys to the second
+        q.normal_(generator=g)
+        kv_indptr[1] = lens[0] - cut
+        out.fill_(0)
+        graph.replay()
+        torch.cuda.synchronize()
+        want, want_lse = torch.empty_like(out), torch.empty_like(lse)
+        call(torch.full_like(ws, 0x5A), want, want_lse)
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), want.view(torch.int16)) and torch.equal(lse, want_lse), i
