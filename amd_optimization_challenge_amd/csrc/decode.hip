@@ -114,7 +114,14 @@ __device__ __forceinline__ void wait_groups(int k) {
 // V block exponent more than kVScaleSpan above E_ref, found so far above its
 // reference anywhere in a pass runs the item again from the maxima of the whole
 // item (nothing of the first pass is kept).  Either way neither the accumulators
-// nor P' of the pass that counts can overflow.
+// nor P' of the pass that counts can overflow.  What the one check costs: a rise
+// early in the item is paid with a whole pass, where the vote per tile stopped at
+// it; what it saves besides the votes is every further pass.  256 x 1024
+// contiguous, mxfp4 / bf16 cache, us a call, vote per tile against this: no rise
+// 36.4 / 57.7 and 29.0 / 57.1, one after the first tile 38.9 / 62.9 and 46.3 / 98.3,
+// one in the last tile 58.2 / 100.8 and 45.0 / 98.4, one at every tile 124 / 441 and
+// 45.1 / 98.4.  (A vote at the second tile alone: 34.1 / 61.7 for the second
+// case, but the contiguous fp4 kernel then spills, 256 x 8192 125.3 -> 130.3.)
 // ============================================================================
 // KF / VF: 0 / 0 fp8 K = V, 1 / 2 fp4 K = V, 1 / 1 fp4 K + fp8 V, 2 / 3 bf16 K =
 // V (a16w16: 1152-byte rows, V = their first 512 dims; QK and PV on 16x16x32
