@@ -579,7 +579,7 @@ int mla_decode_fwd_rows(const void* q_bf16, const void* k_cache, int64_t k_row_s
   p.plan_qlen = q_seq_len;
   e = launch_decode_rows(p, R.grid, s);
   if (e != hipSuccess) return hip_fail(e, "decode launch");
-  e = launch_combine(p, s);
+  e = launch_combine(p, s, true);
   if (e != hipSuccess) return hip_fail(e, "combine launch");
   return MLA_OK;
 }

@@ -1006,7 +1006,9 @@ __global__ __launch_bounds__(256, (H16<KF, VF>::BLOCKS_PER_CU)) void decode_h16_
 // runs four batches side by side (32 pieces of 4 rows: 5.9 -> 4.6 us; at most 8
 // pieces, where the other groups leave at once, as before: 2.4 to 3.8).
 // ============================================================================
-template <int PG>
+// CP: the pieces are the causal rows' (decode_rows.hip), fp16 in 128ths of a cache
+// code; kv_scale enters here.
+template <int PG, bool CP>
 __global__ __launch_bounds__(256 * PG) void combine_kernel(const DecodeParams p) {
   const int b = blockIdx.x, H = p.num_heads;
   const int2 bi = reinterpret_cast<const int2*>(p.plan + kPlanHeader + 4 * p.max_items)[b];
@@ -1050,8 +1052,8 @@ __global__ __launch_bounds__(256 * PG) void combine_kernel(const DecodeParams p)
       const uint32_t wv[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        acc[2 * i] += wg * bf16_bits_to_f32(wv[i] & 0xFFFFu);
-        acc[2 * i + 1] += wg * bf16_bits_to_f32(wv[i] >> 16);
+        acc[2 * i] += wg * (CP ? f16_bits_to_f32(wv[i] & 0xFFFFu) : bf16_bits_to_f32(wv[i] & 0xFFFFu));
+        acc[2 * i + 1] += wg * (CP ? f16_bits_to_f32(wv[i] >> 16) : bf16_bits_to_f32(wv[i] >> 16));
       }
     }
   }
@@ -1082,7 +1084,7 @@ __global__ __launch_bounds__(256 * PG) void combine_kernel(const DecodeParams p)
     }
     M = m;
   }
-  const float inv = wsum > 0.f ? 1.0f / wsum : 0.f;
+  const float inv = (wsum > 0.f ? 1.0f / wsum : 0.f) * (CP ? p.kv_scale[0] * 0.0078125f : 1.f);
   if (p.lse_out != nullptr && blockIdx.z == 0 && (tid & 15) == 0)
     p.lse_out[(int64_t)b * H + head] = wsum > 0.f ? (M + __log2f(wsum)) * kLn2 : neg_inf();
   uint32_t w4[4];
@@ -1157,15 +1159,15 @@ hipError_t launch_decode(const DecodeParams& p, int kv_mode, int grid, hipStream
             : launch_decode_t<false, false>(p, kv_mode, grid, stream);
 }
 
-hipError_t launch_combine(const DecodeParams& p, hipStream_t stream) {
+hipError_t launch_combine(const DecodeParams& p, hipStream_t stream, bool code_pieces) {
   const dim3 grid(p.batch, p.num_heads / 16, 4);
   // up to a block per four CUs (gfx950: 256): rows few enough to be cut into more
   // than 8 pieces; with more blocks 1024-thread ones start later than they save
   // (32 x 1024, 8 pieces: 3.4 us in small blocks, 3.8 in large ones)
-  if (p.batch <= 16 && p.batch * (p.num_heads / 16) * 4 <= 64)
-    hipLaunchKernelGGL((combine_kernel<4>), grid, dim3(1024), 0, stream, p);
-  else
-    hipLaunchKernelGGL((combine_kernel<1>), grid, dim3(256), 0, stream, p);
+  const bool large = p.batch <= 16 && p.batch * (p.num_heads / 16) * 4 <= 64;
+  const auto kernel = large ? (code_pieces ? combine_kernel<4, true> : combine_kernel<4, false>)
+                            : (code_pieces ? combine_kernel<1, true> : combine_kernel<1, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(large ? 1024 : 256), 0, stream, p);
   return hipGetLastError();
 }
 

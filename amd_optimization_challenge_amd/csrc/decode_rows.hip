@@ -409,23 +409,31 @@ __global__ __launch_bounds__(512, 2) void decode_rows_kernel(const DecodeParams 
     }
     return;
   }
-  // a PV wave's 128 dims of every column as bf16 rows in LDS (only it reads
-  // them), then 16-byte row segments
+  // a PV wave's 128 dims of every column as 16-bit rows in LDS (only it reads
+  // them), then 16-byte row segments.  A whole sequence's are the output's bf16.  A
+  // piece's are fp16 in 128ths of a code (at most 448 x 128; the combine brings
+  // kv_scale in): three bits more than bf16 at the same bytes, as this plan cuts
+  // sequences into pieces that row by row stay whole (32 ragged sequences x 4 rows,
+  // error against 64 bits: row by row 2.12e-3, here 2.21e-3 with bf16 pieces)
   uint8_t* ob = smem + w * C::COLS * C::OST;
+  auto stage = [&](float one, auto pack) __attribute__((always_inline)) {
 #pragma unroll
-  for (int ch = 0; ch < 2; ++ch) {
-    const float L = lx[32 * ch + l32] + lx[C::COLS + 32 * ch + l32];
-    const float inv = L > 0.f ? kvs / L : 0.f;
+    for (int ch = 0; ch < 2; ++ch) {
+      const float L = lx[32 * ch + l32] + lx[C::COLS + 32 * ch + l32];
+      const float inv = L > 0.f ? one / L : 0.f;
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const v16f& a = o[ch][e];
-        const uint32_t lo = pack_bf16x2(a[4 * q] * inv, a[4 * q + 1] * inv);
-        const uint32_t hi = pack_bf16x2(a[4 * q + 2] * inv, a[4 * q + 3] * inv);
-        *reinterpret_cast<uint2*>(ob + (32 * ch + l32) * C::OST + 2 * (32 * e + 8 * q + 4 * hh)) = make_uint2(lo, hi);
-      }
-  }
+        for (int q = 0; q < 4; ++q) {
+          const v16f& a = o[ch][e];
+          const uint32_t lo = pack(a[4 * q] * inv, a[4 * q + 1] * inv);
+          const uint32_t hi = pack(a[4 * q + 2] * inv, a[4 * q + 3] * inv);
+          *reinterpret_cast<uint2*>(ob + (32 * ch + l32) * C::OST + 2 * (32 * e + 8 * q + 4 * hh)) = make_uint2(lo, hi);
+        }
+    }
+  };
+  if (slot < 0) stage(kvs, [](float a, float b) __attribute__((always_inline)) { return pack_bf16x2(a, b); });
+  else stage(128.f, [](float a, float b) __attribute__((always_inline)) { return pack_f16x2(a, b); });
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   uint16_t* dst = (slot < 0 ? p.out + (int64_t)b * cols * kVDim : p.part_o + (int64_t)slot * cols * kVDim) + 128 * w;
 #pragma unroll 4

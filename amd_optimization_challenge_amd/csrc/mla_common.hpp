@@ -37,7 +37,7 @@ struct DecodeParams {
   const int32_t* kv_indptr;  // [B+1]
   const int32_t* kv_indices; // [T] or nullptr (identity)
   const int32_t* plan;       // plan block (see above)
-  uint16_t* part_o;          // [max_items, H, 512] bf16 (normalized split outputs)
+  uint16_t* part_o;          // [max_items, H, 512] bf16 (normalized split outputs; decode_rows.hip: fp16, 128 x codes)
   float* part_lse;           // [max_items, H]  (log2 domain)
   uint16_t* out;             // [B, H, 512] bf16
   float* lse_out;            // [B, H] natural-log lse, or nullptr
@@ -105,6 +105,16 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   typedef __bf16 v2bf_t __attribute__((ext_vector_type(2)));
   typedef float v2f_t __attribute__((ext_vector_type(2)));
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f_t{a, b}), v2bf_t));
+}
+
+// two floats -> fp16 pair (RNE), a in the low half; and a half back
+__device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
+  typedef _Float16 v2h_t __attribute__((ext_vector_type(2)));
+  typedef float v2f_t __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((v2f_t{a, b}), v2h_t));
+}
+__device__ __forceinline__ float f16_bits_to_f32(uint32_t h) {
+  return (float)__builtin_bit_cast(_Float16, (uint16_t)h);
 }
 
 // Round-to-nearest-even f32 -> OCP e4m3fn code for |f| <= 448.

@@ -84,7 +84,8 @@ hipError_t launch_append_kv(const uint16_t* x, int64_t n, int64_t x_stride, cons
 
 // decode.hip
 hipError_t launch_decode(const DecodeParams& p, int kv_mode, int grid, hipStream_t stream);
-hipError_t launch_combine(const DecodeParams& p, hipStream_t stream);
+// code_pieces: the pieces are fp16 in 128ths of p.kv_scale's codes (decode_rows.hip), else bf16
+hipError_t launch_combine(const DecodeParams& p, hipStream_t stream, bool code_pieces = false);
 // decode_h128.hip: H = 128 with the fp8 cache
 hipError_t launch_decode_h128f(const DecodeParams& p, int grid, hipStream_t stream);
 hipError_t launch_decode_h128m(const DecodeParams& p, int grid, hipStream_t stream);

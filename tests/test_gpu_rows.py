@@ -120,6 +120,24 @@ def test_huge_scores(log2k, sm, contiguous):
     assert np.allclose(lse.cpu().numpy(), ref_lse, rtol=1e-2)
 
 
+@pytest.mark.parametrize("qlen", [2, 4])
+@pytest.mark.parametrize("outlier", [1.0, 2.0 ** 12])
+def test_pieces_cost_no_precision(qlen, outlier):
+    """Rows in up to eight pieces: 1.66e-3 for the bf16 result and 0.55e-3 for the two
+    fp8 terms of P, 1.75e-3 together in the 2-norm (a bf16 rounding of the pieces would
+    make it 2.2 to 2.35e-3), also where one large value leaves the others small codes."""
+    lens = [260, 300, 400, 513, 600, 777, 900, 1024, 64]
+    q = torch.randn(len(lens) * qlen, 16, 576, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16)
+    _, kv, indptr, idx, _, _ = host_case(lens, 16, "fp8", seed=6)
+    kv = kv.clone()
+    kv[idx[int(indptr[-2])].long(), 0, 3] = 4.0 * outlier  # in the last sequence, left out below
+    case = case_from_tensors(q[:len(lens)], kv, indptr, idx, "fp8")
+    out, _ = _run(case, q, qlen, 0.08)
+    _, ref = O.reference_path(O.bf16_tensor_bits(q), "fp8", case[5], indptr.numpy(), idx.numpy(), 0.08, q_seq_len=qlen)
+    got, ref = out.float().cpu().numpy()[:-qlen], ref[:-qlen]
+    assert np.linalg.norm(got - ref) <= 1.95e-3 * np.linalg.norm(ref)
+
+
 @pytest.mark.parametrize("contiguous", [False, True])
 def test_first_tile_of_minus_infinity(contiguous):
     """Scores of a piece's first tile that overflow to -inf, finite ones after it: the
