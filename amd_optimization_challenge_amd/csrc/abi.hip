@@ -105,11 +105,12 @@ int target_items_for(int batch, int num_heads, int kv_mode, int num_cu) {
 // partials), and from there up the chunk (longest piece) is at least 1024
 // tokens: a two-way split of 1024-token sequences costs more in prologues and
 // partial outputs than the idle slots it fills.  No sequence is cut into more
-// than 32 pieces: the combine folds a sequence's pieces 8 loads at a time per
-// thread, on 4 work-groups per 16 heads, so 64 pieces cost more in that serial
-// tail than the shorter items save.  On the task's shapes (mxfp4 cache, whole
-// call) this took 256 x 1024 from 71 to 61 us, 32 x 8192 from 67 to 64 and
-// 4 x 8192 from 38.5 to 35.9; indexed caches keep target_items_for, their
+// than 32 pieces: a combine that folds a sequence's pieces one batch of 8 after
+// another, on 4 work-groups per 16 heads, lost more to 64 pieces than the shorter
+// items saved.  (Grids of up to 64 blocks fold four batches side by side now; the
+// cap has not been weighed against that form.)  On the task's shapes (mxfp4
+// cache, whole call) this took 256 x 1024 from 71 to 61 us, 32 x 8192 from 67 to
+// 64 and 4 x 8192 from 38.5 to 35.9; indexed caches keep target_items_for, their
 // scattered rows need both slots of a CU in flight (128 x 4096: 97 us at one
 // item per slot, 122 at one per CU).
 PlanTarget plan_target_for(int batch, int num_heads, int kv_mode, int num_cu, bool contiguous) {

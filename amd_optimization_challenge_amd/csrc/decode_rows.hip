@@ -17,7 +17,7 @@
 // doing one after the other, a tile took its whole chain (fragment reads, nine
 // MFMAs, softmax, exchange, sixteen MFMAs), about 2.3 us; side by side 1.2, and
 // 64 keys more of 256 sequences x 4 rows cost what their gather does (6.1 TB/s).
-// The 32 ragged sequences take 24-26 us of decode instead of 48, the call 33.3-35.4
+// The 32 ragged sequences take 24-26 us of decode instead of 48, the call 33.3-35.6
 // instead of 58.0; a third of the rest is start-up (Q of 64 columns quantized, 2 us;
 // the plan, slots and first rows, 4) and 64 KiB of output per item.
 //   Scoring wave w: token half w & 1, column half w >> 1, nine 32x32x64 MFMAs
